@@ -32,6 +32,7 @@ EXPORTS = (
     "launch_gather_probe",
     "launch_sparse_topk_indices",
     "launch_attention_target",
+    "launch_attention_target_split",
     "launch_simple_attention",
     "kernel_config_sparse_mla",
     "kernel_config_attention_target",
@@ -41,6 +42,7 @@ EXPORTS = (
     "kernel_metadata_simple_attention",
     "workspace_size_sparse_mla",
     "workspace_size_attention_target",
+    "workspace_size_attention_target_split",
     "workspace_size_simple_attention",
     "launch_cache_flush",
     "launch_clock_probe",
@@ -101,6 +103,10 @@ _SIGNATURES = {
         [_P] * 6 + [ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
         ct.c_int,
     ),
+    "launch_attention_target_split": (
+        [_P] * 6 + [ct.c_uint64, ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
+        ct.c_int,
+    ),
     "launch_simple_attention": ([_P] * 6 + [ct.c_int64, ct.c_int64], ct.c_int),
     "kernel_config_sparse_mla": ([ct.POINTER(ct.c_int64)], ct.c_int),
     "kernel_config_attention_target": ([ct.POINTER(ct.c_int64)], ct.c_int),
@@ -110,6 +116,10 @@ _SIGNATURES = {
     "kernel_metadata_simple_attention": ([], ct.c_char_p),
     "workspace_size_sparse_mla": ([ct.POINTER(ct.c_uint64), ct.POINTER(SparseMlaParams)], ct.c_int),
     "workspace_size_attention_target": (
+        [ct.POINTER(ct.c_uint64), ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
+        ct.c_int,
+    ),
+    "workspace_size_attention_target_split": (
         [ct.POINTER(ct.c_uint64), ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
         ct.c_int,
     ),

@@ -16,6 +16,9 @@
 // simple_attention: examples/flash_attention/simple.py:60-141. One 128-key
 // tile per head: S = Q K^T * 128^-1/2, P = f16(softmax(S)) normalised BEFORE
 // the cast, O = f16(P V) (simple.py:25-57).
+#include <algorithm>
+#include <cmath>
+
 #include "common.h"
 #include "../../include/ascendflow_amd.h"
 
@@ -372,6 +375,370 @@ __global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
   }
 }
 
+// Flash-attention forward of few query rows per KV head (decode, and prefill
+// grids too small to fill the GPU). The query rows of the HQ / HKV heads that
+// share a KV head are one contiguous block of group * Sq rows of Q and O, so
+// they are packed into tiles of 16 * QT rows and every KV row is read once per
+// tile instead of once per head. A workgroup owns one (batch, KV head, row
+// tile, split): a contiguous range of 32-key tiles, dealt to its four waves in
+// turn. Bound by HBM (each KV byte feeds at most 4 * QT * 16 FLOP per row tile),
+// so the waves are four independent streams with no barrier in the loop: each
+// keeps two K and two V tiles (32 KiB) in flight into an LDS ring of its own
+// and waits on its own load counter only. Each wave holds its own running max,
+// denominator and O over all its keys; they are combined through LDS at the
+// end, and the splits' partial results (FP32) by fa_merge_kernel.
+// STREAM: KV loads are non-temporal, for one or two row tiles whose KV is too
+// large to stay in the 256 MiB Infinity Cache between calls (FD_STREAM_BYTES).
+// Measured, B8 HQ32 HKV8 Sq1 Sk32768 bf16 (1.07 GB of KV), call: 823 -> 160 us
+// (6.7 TB/s) against the forward kernel, whose 256 workgroups of 256 query
+// rows each read their KV head once per query head; B1 HQ32 HKV8 Sq1 Sk16384
+// 389 -> 22 us, B1 HQ32 HKV8 Sq64 Sk8192 207 -> 33 us.
+constexpr int FD_KEYS = 32;                        // keys per tile
+constexpr int FD_TILE = FD_KEYS * 256;             // bytes of one K or V tile
+constexpr int FD_WAVES = 4, FD_SLOTS = 4;          // K, V, K, V of two tiles per wave
+constexpr int FD_LOADS = FD_TILE / 1024;           // wave loads per tile
+constexpr int FD_MAX_QT = 4;
+
+struct FaSplitArgs {
+  FaArgs fa;
+  int32_t group;      // HQ / HKV
+  int32_t row_tiles;  // tiles of 16 * QT rows per (batch, KV head)
+  int32_t splits;
+  float* partial_o;   // [splits][B * HQ * Sq][128], normalised by nothing (relative to its max)
+  float* partial_ml;  // [splits][B * HQ * Sq][2]: running max (log2 units), denominator
+};
+
+template <int DT, int QT, bool STREAM>
+__global__ __launch_bounds__(FD_WAVES * 64, 1) void fa_split_kernel(FaSplitArgs args) {
+  typedef typename B16<DT>::scalar scalar;
+  typedef typename B16<DT>::x8 x8;
+  typedef typename B16<DT>::x4 x4;
+  constexpr int D = 128, ROW_BYTES = 2 * D, UNITS = D / 8, KT = FD_KEYS / 16, ROWS = 16 * QT;
+  const FaArgs& a = args.fa;
+  __shared__ __attribute__((aligned(16))) uint8_t ring[FD_WAVES][FD_SLOTS][FD_TILE];
+  __shared__ float wave_ml[2][FD_WAVES][ROWS];
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int g = lane >> 4, i16 = lane & 15;
+  // Row tiles of one split are neighbours (one XCD: they share its KV rows).
+  const uint32_t logical = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int row_tile = (int)(logical % (uint32_t)args.row_tiles);
+  const uint32_t rest = logical / (uint32_t)args.row_tiles;
+  const int split = (int)(rest % (uint32_t)args.splits);
+  const int64_t kv = rest / (uint32_t)args.splits;  // batch * HKV + KV head
+  const int64_t rows = (int64_t)args.group * a.Sq;  // packed rows of this KV head
+  const int64_t row0 = (int64_t)row_tile * ROWS;    // first one of this tile
+
+  const scalar* Q = (const scalar*)a.q + kv * rows * D;
+  const char* K = (const char*)a.k + kv * a.Sk * ROW_BYTES;
+  const char* V = (const char*)a.v + kv * a.Sk * ROW_BYTES;
+
+  // Keys of the whole tile (causal: up to its largest query), of this split,
+  // and the per-column limit (top-left causal: key j visible to query i iff j <= i).
+  int64_t kv_end = a.Sk, col_limit[QT], clean = a.Sk;
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) col_limit[qt] = a.Sk;
+  if (a.causal) {
+    const int64_t last = min(row0 + ROWS, rows) - 1;
+    // Rows of one head only, in query order, or rows that cross heads (all queries possible).
+    const bool one_head = row0 / a.Sq == last / a.Sq;
+    kv_end = min(a.Sk, (one_head ? last % a.Sq : a.Sq - 1) + 1);
+    clean = min(a.Sk, (one_head ? row0 % a.Sq : 0) + 1);
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) col_limit[qt] = min(a.Sk, (row0 + 16 * qt + i16) % a.Sq + 1);
+  }
+  const int tiles = (int)((kv_end + FD_KEYS - 1) / FD_KEYS);
+  const int first = (int)((int64_t)tiles * split / args.splits), end = (int)((int64_t)tiles * (split + 1) / args.splits);
+  const int n = end - first > wave ? (end - first - wave + FD_WAVES - 1) / FD_WAVES : 0;  // this wave's tiles
+  auto tile_of = [&](int i) { return first + wave + i * FD_WAVES; };
+
+  const uint32_t ring_base = lds_address(ring[wave][0]);
+  auto slot_address = [&](int i, int tensor) {
+    return opaque_uniform(ring_base + (uint32_t)((i & 1) * 2 + tensor) * FD_TILE);
+  };
+  // Wave load p covers rows 4p .. 4p + 3; this lane lands on unit lane % 16 of
+  // row 4p + lane / 16 and loads unit (lane % 16) ^ (row & 15) of that row.
+  uint32_t load_offset[FD_LOADS];
+#pragma unroll
+  for (int p = 0; p < FD_LOADS; ++p) {
+    const int r = 4 * p + lane / UNITS;
+    load_offset[p] = (uint32_t)(r * ROW_BYTES + (((lane % UNITS) ^ (r & 15)) << 4));
+  }
+  auto fetch = [&](int i, int tensor) {
+    const int64_t key0 = (int64_t)tile_of(i) * FD_KEYS;
+    const char* base = (tensor ? V : K) + key0 * ROW_BYTES;
+    const uint32_t dst = slot_address(i, tensor);
+    const bool tail = key0 + FD_KEYS > a.Sk;  // uniform; rows past Sk read the last key instead (masked later)
+#pragma unroll
+    for (int p = 0; p < FD_LOADS; ++p) {
+      uint32_t off = load_offset[p];
+      if (tail) {
+        const int r = 4 * p + lane / UNITS;
+        off = (uint32_t)((int)min((int64_t)r, a.Sk - 1 - key0) * ROW_BYTES + (((lane % UNITS) ^ (r & 15)) << 4));
+      }
+      if constexpr (STREAM)
+        __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                         :: "s"(dst + (uint32_t)p * 1024u), "v"(off), "s"(base) : "memory");
+      else
+        __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         :: "s"(dst + (uint32_t)p * 1024u), "v"(off), "s"(base) : "memory");
+    }
+  };
+
+  x8 qf[QT][D / 32];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const int64_t row = row0 + 16 * qt + i16;
+#pragma unroll
+    for (int j = 0; j < D / 32; ++j)
+      qf[qt][j] = row < rows ? *(const x8*)(Q + row * D + 32 * j + 8 * g) : __builtin_bit_cast(x8, u32x4{0u, 0u, 0u, 0u});
+  }
+  // Q's loads are the wave's oldest and land before the first K tile.
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (i < n) {
+      fetch(i, 0);
+      fetch(i, 1);
+    }
+
+  const int ra = sigma(i16), rt = sigma(4 * g + (i16 >> 2));
+  uint32_t qk_base[D / 32], tr_base[D / 16];
+#pragma unroll
+  for (int j = 0; j < D / 32; ++j) qk_base[j] = (uint32_t)(ra * ROW_BYTES + (((4 * j + g) ^ (ra & 15)) << 4));
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t)
+    tr_base[t] = (uint32_t)(rt * ROW_BYTES + (((2 * t + ((i16 & 3) >> 1)) ^ (rt & 15)) << 4) + (i16 & 1) * 8);
+
+  f32x4 o[QT][D / 16];
+  float m_run[QT], l_run[QT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    m_run[qt] = -1e30f;  // finite: a fully masked tile then gives p = 0, never NaN
+    l_run[qt] = 0.f;
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) o[qt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const float scale_log2 = a.scale * FA_LOG2E;
+
+  // Before tile i the loads in flight are K(i), V(i), K(i+1), V(i+1) as far as
+  // they exist, FD_LOADS each, in that order; K(i+2) replaces K(i) once its
+  // fragments are in registers, then V(i+2) V(i). So K(i), and later V(i), has
+  // landed once at most three younger batches are in flight; in the last two
+  // tiles, which issue nothing, the wait is for everything.
+  static_assert(4 * FD_LOADS < 64, "vmcnt holds 6 bits");
+  for (int i = 0; i < n; ++i) {
+    const bool more = i + 2 < n;
+    if (more)
+      wait_vmcnt<3 * FD_LOADS>();
+    else
+      wait_vmcnt<0>();
+    __asm__ volatile("" ::: "memory");
+    f32x4 s[KT][QT];
+    {
+      const uint32_t tile = slot_address(i, 0);
+      x8 kf[D / 32][KT];
+#pragma unroll
+      for (int j = 0; j < D / 32; ++j)
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+          kf[j][t] = *(const AFA_LDS x8*)(lds_at<uint8_t>(tile + qk_base[j]) + t * 16 * ROW_BYTES);
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) s[t][qt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < D / 32; ++j)
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt) s[t][qt] = B16<DT>::mfma(kf[j][t], qf[qt][j], s[t][qt]);
+    }
+    if (more) {
+      __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);  // K(i) is in registers
+      __asm__ volatile("" ::: "memory");
+      fetch(i + 2, 0);
+    }
+    const int64_t key0 = (int64_t)tile_of(i) * FD_KEYS;
+    if (key0 + FD_KEYS > clean) {  // uniform
+      __asm__ volatile("");
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const int64_t limit = col_limit[qt] - key0;
+        const int lim = limit < 0 ? 0 : (limit > FD_KEYS ? FD_KEYS : (int)limit);
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) s[t][qt][k] = 16 * t + sigma(4 * g + k) < lim ? s[t][qt][k] : -INFINITY;
+      }
+    }
+    float m_new[QT];
+    bool grow = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      float m = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m = fmaxf(m, s[t][qt][k]);
+      m_new[qt] = fmaxf(m_run[qt], max_over_lane_groups(m) * scale_log2);
+      grow |= m_new[qt] > m_run[qt] + fa_tau<DT>();
+    }
+    if (__ballot(grow) != 0ull) {
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const float alpha = fast_exp2(m_run[qt] - m_new[qt]);
+        l_run[qt] *= alpha;
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) o[qt][t] *= alpha;
+        m_run[qt] = m_new[qt];
+      }
+    }
+    x8 pf[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float p = fast_exp2(__builtin_fmaf(s[t][qt][k], scale_log2, -m_run[qt]));
+          sum += p;
+          pf[qt][4 * t + k] = (scalar)p;
+        }
+      l_run[qt] += sum;
+    }
+    if (more) wait_vmcnt<3 * FD_LOADS>();  // else everything landed above
+    __asm__ volatile("" ::: "memory");
+    {
+      const uint32_t tile = slot_address(i, 1);
+      x4 vlo[D / 16], vhi[D / 16];
+#pragma unroll
+      for (int t = 0; t < D / 16; ++t) {
+        const AFA_LDS uint8_t* p = lds_at<uint8_t>(tile + tr_base[t]);
+        vlo[t] = B16<DT>::read_tr((const AFA_LDS void*)p);
+        vhi[t] = B16<DT>::read_tr((const AFA_LDS void*)(p + 16 * ROW_BYTES));
+      }
+#pragma unroll
+      for (int t = 0; t < D / 16; ++t) {
+        const x8 vf = {vlo[t][0], vlo[t][1], vlo[t][2], vlo[t][3], vhi[t][0], vhi[t][1], vhi[t][2], vhi[t][3]};
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) o[qt][t] = B16<DT>::mfma(vf, pf[qt], o[qt][t]);
+      }
+    }
+    if (more) {
+      __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);  // V(i) is in registers
+      __asm__ volatile("" ::: "memory");
+      fetch(i + 2, 1);
+    }
+  }
+
+  // ---- combine the four waves: each scales its O to the common max and lays
+  // it out in its own (now idle) ring as [row][32 units of 4 features], unit u
+  // of row r at u ^ (r & 15).
+  static_assert(ROWS * D * 4 <= FD_SLOTS * FD_TILE, "a wave's O must fit its ring");
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const float l = sum_over_lane_groups(l_run[qt]);
+    if (g == 0) {
+      wave_ml[0][wave][16 * qt + i16] = m_run[qt];
+      wave_ml[1][wave][16 * qt + i16] = l;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    float m = wave_ml[0][0][16 * qt + i16];
+#pragma unroll
+    for (int w = 1; w < FD_WAVES; ++w) m = fmaxf(m, wave_ml[0][w][16 * qt + i16]);
+    const float weight = fast_exp2(m_run[qt] - m);
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t)
+      *(AFA_LDS f32x4*)(uintptr_t)(ring_base + (uint32_t)((16 * qt + i16) * 512 + (((4 * t + g) ^ i16) << 4))) =
+          o[qt][t] * weight;
+  }
+  __syncthreads();
+  // Thread tid takes unit tid % 32 of rows tid / 32, + 8, ...
+  const int u = tid & 31;
+#pragma unroll
+  for (int r = tid >> 5; r < ROWS; r += FD_WAVES * 2) {
+    const int64_t row = row0 + r;
+    if (row >= rows) break;
+    float m = wave_ml[0][0][r];
+#pragma unroll
+    for (int w = 1; w < FD_WAVES; ++w) m = fmaxf(m, wave_ml[0][w][r]);
+    float l = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < FD_WAVES; ++w) {
+      l += wave_ml[1][w][r] * fast_exp2(wave_ml[0][w][r] - m);
+      acc += *lds_at<f32x4>(lds_address(ring[w][0]) + (uint32_t)(r * 512 + ((u ^ (r & 15)) << 4)));
+    }
+    const int64_t out_row = kv * rows + row;
+    if (args.splits == 1) {
+      const float inv = l > 0.f ? 1.0f / l : 0.f;
+      x4 v;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = (scalar)(acc[k] * inv);
+      *(x4*)((scalar*)a.o + out_row * D + 4 * u) = v;
+    } else {
+      const int64_t at = (int64_t)split * (a.B * (int64_t)a.HQ * a.Sq) + out_row;
+      *(f32x4*)(args.partial_o + at * D + 4 * u) = acc;
+      if (u == 0) {
+        args.partial_ml[2 * at] = m;
+        args.partial_ml[2 * at + 1] = l;
+      }
+    }
+  }
+}
+
+// Combines the splits of fa_split_kernel in split order (deterministic): with
+// M = max_s m_s, O = sum_s 2^(m_s - M) O_s / sum_s 2^(m_s - M) l_s. 32 threads
+// per row, four features each.
+constexpr int FM_ROWS = 8;  // rows per workgroup of 256 threads
+template <int DT>
+__global__ __launch_bounds__(256) void fa_merge_kernel(FaSplitArgs args) {
+  typedef typename B16<DT>::scalar scalar;
+  typedef typename B16<DT>::x4 x4;
+  const FaArgs& a = args.fa;
+  const int64_t total = a.B * (int64_t)a.HQ * a.Sq;
+  const int64_t row = (int64_t)blockIdx.x * FM_ROWS + (threadIdx.x >> 5);
+  const int u = threadIdx.x & 31;
+  if (row >= total) return;
+  // Thread u of the row holds the max and denominator of splits u and u + 32.
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    if (u + 32 * k < args.splits) {
+      const float* ml = args.partial_ml + 2 * ((int64_t)(u + 32 * k) * total + row);
+      m[k] = ml[0];
+      l[k] = ml[1];
+    }
+  float M = fmaxf(m[0], m[1]);
+#pragma unroll
+  for (int d = 16; d > 0; d >>= 1) M = fmaxf(M, __shfl_xor(M, d, 32));
+  float w[2], L = 0.f;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    w[k] = u + 32 * k < args.splits ? fast_exp2(m[k] - M) : 0.f;
+    L += w[k] * l[k];
+  }
+#pragma unroll
+  for (int d = 16; d > 0; d >>= 1) L += __shfl_xor(L, d, 32);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const float* src = args.partial_o + row * 128 + 4 * u;
+#pragma unroll 8
+  for (int s = 0; s < args.splits; ++s) {
+    const float ws = __shfl(s < 32 ? w[0] : w[1], s & 31, 32);
+    acc += *(const f32x4*)(src + (int64_t)s * total * 128) * ws;
+  }
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  x4 v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = (scalar)(acc[k] * inv);
+  *(x4*)((scalar*)a.o + row * 128 + 4 * u) = v;
+}
+
 // Teaching attention: one workgroup per (head, 64 query rows), 4 waves of 16
 // queries; the whole 128-key tile is resident, so the softmax is exact and P
 // is normalised before its f16 cast (simple.py:25-41).
@@ -474,6 +841,10 @@ using namespace afa;
 namespace {
 constexpr int FA_NW = 8, FA_QT = 2;
 
+constexpr int FD_MAX_SPLITS = 64;  // fa_merge_kernel keeps two splits per thread of a row
+constexpr int64_t FA_CUS = 256;
+constexpr int64_t FD_STREAM_BYTES = int64_t(128) << 20;
+
 template <int DT>
 int launch_fa(const FaArgs& a, hipStream_t s) {
   constexpr int BQ = FA_NW * FA_QT * 16;
@@ -483,17 +854,120 @@ int launch_fa(const FaArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((fa_forward_kernel<DT, FA_NW, FA_QT>), dim3((unsigned)blocks), dim3(FA_NW * 64), 0, s, a);
   return (int)hipGetLastError();
 }
-}  // namespace
 
-extern "C" int launch_attention_target(void* stream, const void* Q, const void* K, const void* V,
-                                       void* O, void* workspace, int64_t Sq, int64_t Sk,
-                                       const FaParams* p) {
-  (void)workspace;
+// Form of a call: the packed split kernel (qt row tiles of 16 per workgroup,
+// `splits` key ranges) or the forward kernel (qt = 0).
+struct FaPlan {
+  int qt, splits;
+  int64_t row_tiles;
+};
+
+// Picks the cheaper form by a model of MI355X in microseconds (times measured
+// on grids from 16 to 1500 workgroups, bf16), fixed at 256 CUs so that the
+// workspace size depends on the sizes alone. Both kernels run one workgroup
+// per CU:
+//  - forward kernel: FORWARD_STEP per 64-key chunk of a 256-row tile, and
+//    FORWARD_START per workgroup (Q, first loads, output);
+//  - split kernel: a step of four 32-key tiles costs the larger of
+//    SPLIT_STEP[qt] (the latency of 64 KiB of loads, then the waves' own chain
+//    of MFMAs and softmax) and KV_STEP, its 64 KiB when all CUs load at once
+//    (6.9 TB/s), shared by the row tiles that read the same keys; SPLIT_START
+//    for the first workgroup of a CU, ROUND + ROUND_QT * qt for each later one
+//    (its first loads, and the waves' O through LDS), MERGE + MERGE_SPLIT
+//    per split for the second kernel.
+// A causal grid runs at least its longest tile and at most twice the mean.
+// Measured either side of the line (us, split / forward kernel): B1 HQ8 Sq1024
+// causal 18.4 / 36.6, B1 HQ32 HKV8 Sq1000 causal 56 / 37, B1 HQ32 HKV8 Sq256
+// Sk8192 96 / 224, B1 HQ32 HKV8 Sq2000 193 / 73.
+// with_splits: there is a workspace for partial results.
+FaPlan choose_fa(const FaArgs& a, bool with_splits) {
+  constexpr double FORWARD_STEP = 1.65, FORWARD_START = 8.0;
+  constexpr double KV_STEP = 2.4, SPLIT_START = 10.0, ROUND = 3.0, ROUND_QT = 1.6, MERGE = 3.0, MERGE_SPLIT = 0.12;
+  constexpr double SPLIT_STEP[FD_MAX_QT + 1] = {0, 1.4, 1.55, 2.0, 2.45};
+  const int64_t group = a.HQ / a.HKV, kv_heads = (int64_t)a.B * a.HKV, rows = group * a.Sq;
+  const int64_t keys = a.causal ? std::min(a.Sk, a.Sq) : a.Sk;
+  // Time of `blocks` workgroups whose longest takes `steps` steps.
+  auto grid_cost = [&](int64_t blocks, int64_t row_tiles_per_head, double steps, double step, double round) {
+    const double rounds = std::ceil((double)blocks / FA_CUS);
+    const double mean = a.causal && row_tiles_per_head > 1 ? 0.5 * (1 + 1.0 / row_tiles_per_head) : 1.0;
+    return (rounds - 1) * round + std::max(1.0, rounds * mean) * steps * step;
+  };
+  const int64_t forward_tiles = (a.Sq + 255) / 256;
+  FaPlan plan{0, 1, 0};
+  double best = FORWARD_START + grid_cost(forward_tiles * a.B * a.HQ, forward_tiles, std::ceil(keys / 64.0),
+                                          FORWARD_STEP, FORWARD_START);
+  for (int qt = 1; qt <= FD_MAX_QT; ++qt) {
+    const int64_t row_tiles = (rows + 16 * qt - 1) / (16 * qt);
+    if (qt > 1 && rows <= 16 * (qt - 1)) break;  // no fewer tiles than with qt - 1
+    const int64_t items = kv_heads * row_tiles;
+    if (items * FD_MAX_SPLITS > 0x7fffffffLL) continue;
+    // A causal row tile that crosses heads walks every key of both: only where those are few.
+    if (a.causal && group > 1 && a.Sq > 256 && a.Sq % (16 * qt)) continue;
+    const int64_t key_tiles = (keys + FD_KEYS - 1) / FD_KEYS;
+    const int64_t most = with_splits ? std::min<int64_t>(FD_MAX_SPLITS, std::max<int64_t>(1, key_tiles / FD_WAVES)) : 1;
+    for (int64_t splits = 1; splits <= most; ++splits) {
+      const int64_t blocks = items * splits;
+      const double active = std::min<double>(1.0, (double)blocks / FA_CUS);
+      const double steps = std::ceil((double)key_tiles / splits / FD_WAVES);
+      const double cost = SPLIT_START + (splits > 1 ? MERGE + MERGE_SPLIT * splits : 0.0) +
+                          grid_cost(blocks, (a.Sq + 16 * qt - 1) / (16 * qt), steps,
+                                    std::max(SPLIT_STEP[qt], KV_STEP * active / row_tiles), ROUND + ROUND_QT * qt);
+      if (cost < best) {
+        best = cost;
+        plan = FaPlan{qt, (int)splits, row_tiles};
+      }
+    }
+  }
+  return plan;
+}
+
+int64_t fa_split_bytes(const FaArgs& a, const FaPlan& plan) {
+  return plan.splits > 1 ? (int64_t)plan.splits * a.B * a.HQ * a.Sq * (128 + 2) * 4 : 0;
+}
+
+template <int DT>
+int launch_split(const FaArgs& a, const FaPlan& plan, void* workspace, hipStream_t s) {
+  FaSplitArgs args;
+  args.fa = a;
+  args.group = a.HQ / a.HKV;
+  args.row_tiles = (int32_t)plan.row_tiles;
+  args.splits = plan.splits;
+  const int64_t total = (int64_t)a.B * a.HQ * a.Sq;
+  args.partial_o = (float*)workspace;
+  args.partial_ml = (float*)workspace + plan.splits * total * 128;
+  const dim3 grid((unsigned)((int64_t)a.B * a.HKV * plan.row_tiles * plan.splits)), block(FD_WAVES * 64);
+  // Non-temporal KV loads, measured with and without (us): 1.07 GB of KV 160 /
+  // 182, 268 MB 46.8 / 52.8, 134 MB 27.9 / 31.2; but 67 MB, part of which stays
+  // cached between calls, 24.0 / 21.7. Calls of three row tiles and more share
+  // their KV through the L2 (262 MB 100.1 / 99.6) and keep ordinary loads.
+  const bool stream = plan.row_tiles <= 2 && 2 * 256 * (int64_t)a.B * a.HKV * a.Sk >= FD_STREAM_BYTES;
+  if (stream && plan.qt == 1)
+    hipLaunchKernelGGL((fa_split_kernel<DT, 1, true>), grid, block, 0, s, args);
+  else if (stream && plan.qt == 2)
+    hipLaunchKernelGGL((fa_split_kernel<DT, 2, true>), grid, block, 0, s, args);
+  else if (plan.qt == 1)
+    hipLaunchKernelGGL((fa_split_kernel<DT, 1, false>), grid, block, 0, s, args);
+  else if (plan.qt == 2)
+    hipLaunchKernelGGL((fa_split_kernel<DT, 2, false>), grid, block, 0, s, args);
+  else if (plan.qt == 3)
+    hipLaunchKernelGGL((fa_split_kernel<DT, 3, false>), grid, block, 0, s, args);
+  else
+    hipLaunchKernelGGL((fa_split_kernel<DT, 4, false>), grid, block, 0, s, args);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || plan.splits == 1) return (int)e;
+  hipLaunchKernelGGL(fa_merge_kernel<DT>, dim3((unsigned)((total + FM_ROWS - 1) / FM_ROWS)), dim3(256), 0, s, args);
+  return (int)hipGetLastError();
+}
+
+int check_fa(int64_t Sq, int64_t Sk, const FaParams* p) {
   if (!p) return AFA_E_NULL;
-  if (!Q || !K || !V || !O) return AFA_E_NULL;
   if (p->dtype != AFA_DTYPE_BF16 && p->dtype != AFA_DTYPE_F16) return AFA_E_DTYPE;
   if (p->D != 128 || p->B <= 0 || p->HQ <= 0 || p->HKV <= 0 || p->HQ % p->HKV) return AFA_E_SHAPE;
   if (Sq < 1 || Sk < 1 || !(p->scale > 0.0f)) return AFA_E_SHAPE;
+  return AFA_OK;
+}
+
+FaArgs make_fa(const void* Q, const void* K, const void* V, void* O, int64_t Sq, int64_t Sk, const FaParams* p) {
   FaArgs a;
   a.q = Q;
   a.k = K;
@@ -506,8 +980,49 @@ extern "C" int launch_attention_target(void* stream, const void* Q, const void* 
   a.HKV = p->HKV;
   a.causal = p->causal ? 1 : 0;
   a.scale = p->scale;
-  hipStream_t s = (hipStream_t)stream;
-  return p->dtype == AFA_DTYPE_F16 ? launch_fa<DT_F16>(a, s) : launch_fa<DT_BF16>(a, s);
+  return a;
+}
+
+int dispatch_fa(const FaArgs& a, const FaPlan& plan, void* workspace, int dtype, hipStream_t s) {
+  if (plan.qt == 0) return dtype == AFA_DTYPE_F16 ? launch_fa<DT_F16>(a, s) : launch_fa<DT_BF16>(a, s);
+  return dtype == AFA_DTYPE_F16 ? launch_split<DT_F16>(a, plan, workspace, s)
+                                : launch_split<DT_BF16>(a, plan, workspace, s);
+}
+}  // namespace
+
+extern "C" int launch_attention_target(void* stream, const void* Q, const void* K, const void* V,
+                                       void* O, void* workspace, int64_t Sq, int64_t Sk,
+                                       const FaParams* p) {
+  (void)workspace;
+  if (!p) return AFA_E_NULL;
+  if (!Q || !K || !V || !O) return AFA_E_NULL;
+  const int status = check_fa(Sq, Sk, p);
+  if (status) return status;
+  const FaArgs a = make_fa(Q, K, V, O, Sq, Sk, p);
+  return dispatch_fa(a, choose_fa(a, false), nullptr, p->dtype, (hipStream_t)stream);
+}
+
+extern "C" int workspace_size_attention_target_split(uint64_t* bytes, int64_t Sq, int64_t Sk, const FaParams* p) {
+  if (!bytes) return -1;
+  const int status = check_fa(Sq, Sk, p);
+  if (status) return status;
+  const FaArgs a = make_fa(nullptr, nullptr, nullptr, nullptr, Sq, Sk, p);
+  *bytes = (uint64_t)fa_split_bytes(a, choose_fa(a, true));
+  return AFA_OK;
+}
+
+extern "C" int launch_attention_target_split(void* stream, const void* Q, const void* K, const void* V, void* O,
+                                             void* workspace, uint64_t workspace_bytes, int64_t Sq, int64_t Sk,
+                                             const FaParams* p) {
+  if (!p) return AFA_E_NULL;
+  if (!Q || !K || !V || !O) return AFA_E_NULL;
+  const int status = check_fa(Sq, Sk, p);
+  if (status) return status;
+  const FaArgs a = make_fa(Q, K, V, O, Sq, Sk, p);
+  const FaPlan plan = choose_fa(a, true);
+  const int64_t need = fa_split_bytes(a, plan);
+  if (need > 0 && (!workspace || workspace_bytes < (uint64_t)need)) return AFA_E_WORKSPACE;
+  return dispatch_fa(a, plan, workspace, p->dtype, (hipStream_t)stream);
 }
 
 extern "C" int launch_simple_attention(void* stream, const void* Q, const void* K, const void* V,

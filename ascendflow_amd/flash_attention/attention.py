@@ -2,8 +2,10 @@
 
 Drop-in for ``examples/flash_attention/attention.py:243-264`` (``attention_target``)
 and its host tiling policy ``causal_policy`` (``attention.py:19-26``). The call
-launches the fused gfx950 kernel of ``csrc/flash_attention.hip`` through
-``launch_attention_target`` on the current stream. The Ascend tiling
+launches the gfx950 kernels of ``csrc/flash_attention.hip`` through
+``launch_attention_target_split`` on the current stream: one fused kernel, or,
+for few query rows and small grids, a kernel over split keys and the merge of
+its partial results. The Ascend tiling
 constexprs (BQ, BM, BK, CK, VR, GROUPS) are checked against the reference's
 asserts (``attention.py:305-318``) and otherwise ignored.
 """
@@ -11,6 +13,9 @@ asserts (``attention.py:305-318``) and otherwise ignored.
 from __future__ import annotations
 
 import ctypes as ct
+import functools
+
+import torch
 
 from .. import _native
 from .._tensors import DTYPES, check_disjoint, check_tensor, require, storage_dtype, stream_handle
@@ -24,6 +29,18 @@ def causal_policy(sq, sk):
     if prefix < 8192:
         return {"kv_tile": 512, "vector_rows": 16}
     return {"kv_tile": 1024, "vector_rows": 8}
+
+
+@functools.lru_cache(maxsize=64)
+def _launch_state(lib, B, HQ, HKV, D, dtype, causal, scale, Sq, Sk):
+    """Launcher parameters and workspace bytes of one set of sizes (neither changes afterwards)."""
+    params = _native.FaParams(
+        B=B, HQ=HQ, HKV=HKV, D=D, dtype=_native.AFA_DTYPE[dtype], causal=int(causal), scale=scale, reserved=0
+    )
+    nbytes = ct.c_uint64(0)
+    _native.check(lib.workspace_size_attention_target_split(ct.byref(nbytes), Sq, Sk, ct.byref(params)),
+                  "workspace_size_attention_target_split")
+    return ct.pointer(params), nbytes.value
 
 
 def attention_target(
@@ -64,11 +81,13 @@ def attention_target(
     check_tensor("V", V, (B, HKV, Sk, D), b16, Q.device)
     check_tensor("O", O, (B, HQ, Sq, D), b16, Q.device)
     check_disjoint([("Q", Q, False), ("K", K, False), ("V", V, False), ("O", O, True)])
-    params = _native.FaParams(
-        B=B, HQ=HQ, HKV=HKV, D=D, dtype=_native.AFA_DTYPE[dtype], causal=int(bool(CAUSAL)), scale=SCALE, reserved=0
+    lib = _native.library()
+    params, nbytes = _launch_state(lib, B, HQ, HKV, D, dtype, bool(CAUSAL), SCALE, Sq, Sk)
+    # Partial results of split keys; the caching allocator keeps the block for this stream.
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=Q.device) if nbytes else None
+    status = lib.launch_attention_target_split(
+        stream_handle(Q.device), Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(),
+        None if workspace is None else workspace.data_ptr(), nbytes, Sq, Sk, params
     )
-    status = _native.library().launch_attention_target(
-        stream_handle(Q.device), Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(), None, Sq, Sk, ct.byref(params)
-    )
-    _native.check(status, "launch_attention_target")
+    _native.check(status, "launch_attention_target_split")
     return O

@@ -163,6 +163,20 @@ typedef struct FaParams {
 int launch_attention_target(void* stream, const void* Q, const void* K, const void* V, void* O,
                             void* workspace, int64_t Sq, int64_t Sk, const FaParams* params);
 
+/* Flash attention with a workspace for calls of few query rows (decode) or
+ * grids too small for the GPU: the keys are split over workgroups, whose FP32
+ * partial results (per split: B * HQ * Sq rows of 128 + 2 floats) a second
+ * kernel combines in split order. workspace_size_attention_target_split gives
+ * the bytes a call needs (0 where one kernel does it, and then `workspace` may
+ * be NULL); the launcher returns AFA_E_WORKSPACE, before any launch, for less.
+ * The same results as launch_attention_target up to FP32 summation order, and
+ * the same arguments accepted. launch_attention_target itself never splits. No
+ * counterpart in the reference, whose operator is one kernel. */
+int workspace_size_attention_target_split(uint64_t* bytes, int64_t Sq, int64_t Sk, const FaParams* params);
+int launch_attention_target_split(void* stream, const void* Q, const void* K, const void* V, void* O,
+                                  void* workspace, uint64_t workspace_bytes, int64_t Sq, int64_t Sk,
+                                  const FaParams* params);
+
 /* Teaching attention: examples/flash_attention/simple.py:60-141.
  *   Q [H,S,128] f16, K/V [H,128,128] f16, O [H,S,128] f16 (written);
  * softmax(QK^T / sqrt(128)) normalised before the f16 cast of P. */
