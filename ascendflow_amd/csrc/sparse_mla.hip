@@ -10,8 +10,8 @@
 //   1. resolve the token's request and window/compressed bounds
 //      (gather.py:8-35, attention.py:339-341) and compact every selected row
 //      (window positions, then compressed ranks, duplicates kept) into an LDS
-//      row list of physical row ids. With a workspace and at least two work
-//      items per CU, a plan kernel does this for every token first and a
+//      row list of physical row ids. At D = 512, with a workspace and at least
+//      two work items per CU, a plan kernel does this for every token first and a
 //      persistent form (sparse_mla_persistent_kernel) streams the tokens of
 //      each CU through one pipeline, so the dependent global round trips
 //      and the pipeline fill no longer idle the matrix cores at token starts;
@@ -80,6 +80,7 @@ struct SparseArgs {
   int32_t split_from;    // first split (token, head tile) key; keys below it run whole
   int32_t ring;          // KV ring tiles of the persistent kernel (3 or 4)
   int32_t stream_kv;     // few query tokens per request: non-temporal KV, Q and O accesses (D = 512)
+  int32_t write_plan;    // one-item kernel: leave the row lists in plan_count / plan_rows
   float scale;
 };
 
@@ -558,6 +559,15 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
       }
     }
     block_barrier();
+    if constexpr (D != 512) {
+      if (a.write_plan && head0 == 0) {
+        // The plan as sparse_plan_kernel writes it. These stores only make the
+        // load waits below stricter: vmcnt counts them too.
+        uint32_t* dst = a.plan_rows + (size_t)token * a.list_pad;
+        for (int r = tid; r < max(padded, CHUNK); r += NT) dst[r] = n_rows > 0 ? row_list[r] : 0u;
+        if (tid == 0) a.plan_count[token] = n_rows;
+      }
+    }
   }
   // This item's list chunks: all of them, or its part's range (an empty part
   // streams one fully masked chunk of list chunk 0).
@@ -1637,6 +1647,7 @@ static SparseArgs make_args(const SparseMlaParams* p, const void* q, const void*
   a.list_pad = (p->WINDOW + p->TOPK + 255) / 256 * 256;
   a.plan_rows = nullptr;
   a.plan_count = nullptr;
+  a.write_plan = 0;
   a.partials = nullptr;
   const Split split = choose_split(p);
   a.parts = split.parts;
@@ -1753,23 +1764,32 @@ static int after_one_item(const SparseArgs& a, int64_t tiles, hipStream_t stream
 }
 
 template <int DT, int D, int NQ, int NP>
-static int launch_fused(const SparseArgs& a, hipStream_t stream) {
+static int launch_fused(SparseArgs a, hipStream_t stream) {
   const size_t lds = (size_t)a.list_pad * sizeof(uint32_t);
   const int64_t tiles = (int64_t)a.T * (a.H / a.BM);
-  if (a.plan_rows != nullptr && a.parts == 1) {
-    // Plan kernel, then the persistent kernel over the plan when every CU gets
-    // at least two items (the persistent form removes the per-item start,
-    // which outweighs a second kernel only then) and a KV ring with its
-    // row-list ring fits. Otherwise (and for split keys) the
-    // one-item-per-workgroup kernel resolves its own rows.
-    static const int cus = device_cus();
-    const int ring = persistent_ring<DT, D, NQ, NP>(a);
-    if (tiles >= 2 * (int64_t)cus && ring != 0) {
-      constexpr int PLAN_THREADS = 64;
-      hipLaunchKernelGGL((sparse_plan_kernel<PLAN_THREADS>), dim3((unsigned)a.T), dim3(PLAN_THREADS), lds, stream, a);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return (int)e;
-      return launch_persistent<DT, D, NQ, NP>(a, ring, stream);
+  static const int cus = device_cus();
+  if (a.plan_rows != nullptr && a.parts == 1 && tiles >= 2 * (int64_t)cus) {
+    // Two items per CU and more, unsplit: the plan stays in the workspace.
+    // D = 512, where one workgroup fills a CU: plan kernel, then the persistent
+    // kernel over the plan (it removes the per-item start, which outweighs a
+    // second kernel), where a KV ring with its row-list ring fits. Smaller D:
+    // two or three workgroups of the one-item kernel share a CU and hide each
+    // other's start, and it leaves the plan itself; measured against plan +
+    // persistent (one workgroup per CU / the best of one to three, us): 1403
+    // tokens of 32 heads x 256 f16 66 / 112 / 77, 8000 bf16 348 / 655 / 361;
+    // 2000 of 64 heads x 256 102 / 142 / 142; of 64 heads x 128 4000 122 / 209
+    // / 141, 640 24.5 / 46.7 / 37.2.
+    if constexpr (D == 512) {
+      const int ring = persistent_ring<DT, D, NQ, NP>(a);
+      if (ring != 0) {
+        constexpr int PLAN_THREADS = 64;
+        hipLaunchKernelGGL((sparse_plan_kernel<PLAN_THREADS>), dim3((unsigned)a.T), dim3(PLAN_THREADS), lds, stream, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+        return launch_persistent<DT, D, NQ, NP>(a, ring, stream);
+      }
+    } else {
+      a.write_plan = 1;
     }
   }
   // One workgroup per item (whole keys, then the parts of split keys): a

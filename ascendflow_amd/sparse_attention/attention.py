@@ -306,7 +306,7 @@ def sparse_mla(*args, **kwargs):
     that shortens the longest per-CU stream (decode-sized batches).
 
     ``ring`` (optional, 3 or 4) fixes the KV ring of the persistent kernel on
-    the plan path: 3 tiles of 32 rows (one chunk in flight) or 4 (two, where
+    the plan path at D = 512: 3 tiles of 32 rows (one chunk in flight) or 4 (two, where
     the row lists fit next to them). By default 4 when ``ori_kv`` and
     ``cmp_kv`` together exceed the 256 MiB Infinity Cache, else 3. The output
     does not depend on it.

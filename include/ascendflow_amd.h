@@ -96,9 +96,10 @@ typedef struct SparseMlaParams {
  *   ori_topk_length i32 [T,1], sinks f32 [H], attention_out [T,H,D] (written).
  * `workspace`: NULL, or at least workspace_size_sparse_mla() bytes of device
  * memory that the call may overwrite. With a workspace and at least two work
- * items (token x BM-head tile) per compute unit, a plan kernel first writes
- * every token's selected-row list into it and a persistent attention kernel
- * streams the items of each compute unit over those lists. The plan is:
+ * items (token x BM-head tile) per compute unit, the call leaves every token's
+ * selected-row list in it: at D = 512 a plan kernel writes them first and a
+ * persistent attention kernel streams the items of each compute unit over
+ * them, at smaller D the one-workgroup-per-item kernel writes what it resolves. The plan is:
  * int32 counts [T] at byte 0 (selected rows per token), then, from byte
  * round_up(4 T, 256), uint32 lists [T][round_up(WINDOW + TOPK, 256)] of
  * tagged rows (bit 31 set: cmp_kv row, else ori_kv row; physical row in the
