@@ -31,6 +31,8 @@ EXPORTS = (
     "launch_sparse_mla_planned",
     "launch_gather_probe",
     "launch_sparse_topk_indices",
+    "launch_sparse_topk_indices_split",
+    "workspace_size_sparse_topk_indices_split",
     "launch_attention_target",
     "launch_attention_target_split",
     "launch_simple_attention",
@@ -99,6 +101,8 @@ _SIGNATURES = {
         ct.c_int,
     ),
     "launch_sparse_topk_indices": ([_P] * 7, ct.c_int),
+    "launch_sparse_topk_indices_split": ([_P] * 7 + [ct.c_uint64, _P], ct.c_int),
+    "workspace_size_sparse_topk_indices_split": ([ct.POINTER(ct.c_uint64), _P], ct.c_int),
     "launch_attention_target": (
         [_P] * 6 + [ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
         ct.c_int,

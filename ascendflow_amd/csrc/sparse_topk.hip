@@ -11,8 +11,10 @@
 // every token, the min(TOPK, C_b, cutoff) positions of largest score among
 // [0, cutoff), ties to the lower position, in ascending order.
 //
-// One workgroup per token; the selection works on a monotonic 32-bit key of
-// each score. sparse_topk_filter (rows up to 256K positions; 256 threads up
+// The selection works on a monotonic 32-bit key of each score. Three kernels:
+// sparse_topk_row keeps a row in registers (calls of few tokens, rows up to 32K
+// positions; longer ones split into segments and merged), described at its
+// definition; the other two stream a row per workgroup. sparse_topk_filter (rows up to 256K positions; 256 threads up
 // to 32K positions, 1024 beyond):
 //   1. sample: four keys per thread (two in the 1024-thread form: 2048
 //      keys), in blocks of 16 consecutive positions
@@ -40,6 +42,7 @@
 // The row is read once from HBM on the common path. sparse_topk_stream
 // serves longer rows: every digit, and the output, re-read the row.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 #include "../../include/ascendflow_amd.h"
@@ -84,6 +87,11 @@ struct TopkArgs {
   int32_t B, T, TOPK, RATIO;
   int32_t cap;              // filter buffer entries (dynamic LDS)
   int32_t words;            // bitmap words per row in dynamic LDS: ceil(C / 32)
+  int32_t first_token;      // token of workgroup 0 (sparse_topk_row)
+  int32_t segments;         // of a split row (sparse_topk_row)
+  int32_t seg_keep;         // entries kept per segment: min(TOPK, segment) rounded up to 4
+  uint32_t* seg_key;        // workspace: [tokens][segments][seg_keep] keys, 0 for none
+  int32_t* seg_pos;         // workspace: [tokens][segments][seg_keep] positions
 };
 
 // Candidates [0, cand) of a token and how many of them it takes, after the
@@ -171,7 +179,7 @@ template <bool PACKED>
 struct RadixLds {
   static constexpr int WORDS = PACKED ? TK_BINS / 2 : TK_BINS;
   alignas(16) uint32_t hist[2][WORDS];
-  int choice[2];  // bin of the digit, keys in the bins above it
+  int choice[3];  // bin of the digit, keys in the bins above it, keys in it (pick_bin)
   __device__ __forceinline__ void add(int parity, int bin, int n) {
     if constexpr (PACKED)
       atomicAdd(&hist[parity][bin >> 1], (uint32_t)n << ((bin & 1) * 16));
@@ -185,6 +193,54 @@ struct RadixLds {
       return (int)hist[parity][bin];
   }
 };
+
+// One wave: the bin of histogram lds.hist[cur] holding the need-th largest
+// entry, into lds.choice (bin, entries in the bins above it). ROW: also the
+// entries in it, and where there are fewer than `need` the lowest bin.
+template <bool PACKED, bool ROW = false>
+__device__ __forceinline__ void pick_bin(RadixLds<PACKED>& lds, int cur, int bins, int need, int lane) {
+  // Lane l sums bins [bins - (l + 1) per, bins - l per): U = 2, 4 or 8
+  // aligned 16-byte units of whole words, read in the order c, c + 1, ...
+  // (mod U) with c chosen so that the 16 lanes one ds_read_b128 pass
+  // serves (four quads whose (lane >> 3) & 3 differ) touch 16 distinct
+  // bank groups. Packed words are summed whole: no half-word sum reaches
+  // 2^16. The lane whose bins hold the need-th key is found by a scan over
+  // the lanes, then its bins are read one per lane and scanned the same way.
+  const int per = bins / 64;
+  const int W = PACKED ? per / 2 : per, U = W / 4;
+  const int quad = (lane >> 3) & 3;
+  const int c = U == 2 ? (quad & 1) : U == 4 ? quad : (((lane >> 1) & 1) | (quad << 1));
+  const uint32_t* words = lds.hist[cur] + (bins - (lane + 1) * per) / (PACKED ? 2 : 1);
+  uint32_t sum = 0;
+#pragma unroll
+  for (int it = 0; it < 8; ++it) {
+    if (it < U) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(words + 4 * ((c + it) & (U - 1)));
+      sum += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+  }
+  const int local = PACKED ? (int)((sum & 0xffffu) + (sum >> 16)) : (int)sum;
+  const int incl = wave_inclusive_scan(local);
+  const uint64_t holds = __ballot(incl - local < need && incl >= need);
+  if (ROW && holds == 0) {
+    if (lane == 0) {
+      lds.choice[0] = 0;
+      lds.choice[1] = 0;
+      lds.choice[2] = need;
+    }
+    return;
+  }
+  const int owner = (int)__builtin_ctzll(holds);
+  const int above = __builtin_amdgcn_readlane(incl - local, owner);  // owner is wave-uniform
+  const int count = lane < per ? lds.get(cur, bins - 1 - (owner * per + lane)) : 0;
+  const int incl2 = wave_inclusive_scan(count);
+  const int q = (int)__builtin_ctzll(__ballot(lane < per && above + incl2 >= need));
+  if (lane == q) {
+    lds.choice[0] = bins - 1 - (owner * per + q);
+    lds.choice[1] = above + incl2 - count;
+    if constexpr (ROW) lds.choice[2] = count;
+  }
+}
 
 // Radix selection of the rank-th largest key among those a key source
 // yields: for_each_key(f) calls f(key) for every key of the source held by
@@ -223,37 +279,7 @@ __device__ __forceinline__ uint32_t radix_select(ForEachKey for_each_key, int ra
     });
     __syncthreads();
     if (tid < 64) {
-      // Lane l sums bins [bins - (l + 1) per, bins - l per): U = 2, 4 or 8
-      // aligned 16-byte units of whole words, read in the order c, c + 1, ...
-      // (mod U) with c chosen so that the 16 lanes one ds_read_b128 pass
-      // serves (four quads whose (lane >> 3) & 3 differ) touch 16 distinct
-      // bank groups. Packed words are summed whole: no half-word sum reaches
-      // 2^16. The lane whose bins hold the need-th key is found by a scan over
-      // the lanes, then its bins are read one per lane and scanned the same way.
-      const int per = bins / 64;
-      const int W = PACKED ? per / 2 : per, U = W / 4;
-      const int quad = (lane >> 3) & 3;
-      const int c = U == 2 ? (quad & 1) : U == 4 ? quad : (((lane >> 1) & 1) | (quad << 1));
-      const uint32_t* words = lds.hist[cur] + (bins - (lane + 1) * per) / (PACKED ? 2 : 1);
-      uint32_t sum = 0;
-#pragma unroll
-      for (int it = 0; it < 8; ++it) {
-        if (it < U) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(words + 4 * ((c + it) & (U - 1)));
-          sum += (v[0] + v[1]) + (v[2] + v[3]);
-        }
-      }
-      const int local = PACKED ? (int)((sum & 0xffffu) + (sum >> 16)) : (int)sum;
-      const int incl = wave_inclusive_scan(local);
-      const int owner = (int)__builtin_ctzll(__ballot(incl - local < need && incl >= need));
-      const int above = __builtin_amdgcn_readlane(incl - local, owner);  // owner is wave-uniform
-      const int count = lane < per ? lds.get(cur, bins - 1 - (owner * per + lane)) : 0;
-      const int incl2 = wave_inclusive_scan(count);
-      const int q = (int)__builtin_ctzll(__ballot(lane < per && above + incl2 >= need));
-      if (lane == q) {
-        lds.choice[0] = bins - 1 - (owner * per + q);
-        lds.choice[1] = above + incl2 - count;
-      }
+      pick_bin<PACKED>(lds, cur, bins, need, lane);
     } else {
       uint32_t* spare = lds.hist[parity ^ 1];
       for (int i = 4 * (tid - 64); i < RadixLds<PACKED>::WORDS; i += 4 * (THREADS - 64))
@@ -604,6 +630,405 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
   }
 }
 
+// ---- rows held in registers --------------------------------------------------
+//
+// sparse_topk_row: one workgroup selects from up to THREADS * ITEMS positions
+// that it keeps in registers: one 16-byte load per group of four positions, all
+// in flight at once and in one round trip with the request lookup's. What bounds
+// it is the chain of dependent steps of one row (calls of few tokens) and the
+// vector operations per score (many): a score costs its key, a maximum, a
+// comparison and a count.
+//   1. bound: at least `take` scores are no smaller than the take-th largest
+//      group maximum, so that is a lower bound of the threshold, and a close one
+//      while groups outnumber `take` (512 of 16K: about 540 scores reach it). No
+//      sample can miss it, so no row is filtered twice. It is taken to the
+//      resolution of one histogram, linear in the score between the smallest
+//      and largest finite maximum: the leading digit of the float key, which
+//      crowds most of a row into a few bins, would take two.
+//   2. keys that reach the bound go to LDS with their positions, in position
+//      order (counts per group and wave, one scan);
+//   3. the threshold among them: one linear histogram, whose bin of the
+//      take-th key holds few; those are ranked against each other (more than
+//      SMALL of them: radix selection);
+//   4. the entries that are taken, compacted in order, are the output.
+// A row with no usable range (its finite maxima all equal, or none finite) or
+// with more entries than LDS holds (many equal scores; TOPK above about half
+// of TK_ENTRIES) takes the radix selection over the whole row, read again.
+// Measured, call (us, against the streaming forms): 64 rows of 16K 29.8 -> 16,
+// 300 31.5 -> 16, 2000 56.7 -> 40.3, 4096 82.6 -> 72.5; 300 rows of 30K 68.4 ->
+// 20; split, 4 rows of 256K 66 -> 22, of 512K 2,500 -> 22. One 16K row in a
+// 1024-thread workgroup takes 8.2 us: row and lookup 3.3, bound 1.3, entries 1.6,
+// threshold 1.6, output 0.4.
+//
+// ROW: scores to indices. SEGMENT: blockIdx.y is a segment of a longer row;
+// its min(TOPK, candidates) largest go to the workspace as keys and positions
+// in ascending position order, then key 0 up to a.seg_keep entries. MERGE: the
+// segments' entries of a token, in order, are the row (their order is the
+// position order, so ties resolve alike), and give the indices.
+enum { TK_ROW = 0, TK_SEGMENT = 1, TK_MERGE = 2 };
+constexpr int TK_ENTRIES = 2048;  // keys that reach the bound, at most
+constexpr uint32_t KEY_LOWEST = 0x00800000u, KEY_HIGHEST = 0xff7fffffu;  // keys of -FLT_MAX and FLT_MAX
+
+__device__ __forceinline__ float key_score(uint32_t k) {  // inverse of score_key, of the nearest finite key
+  k = min(max(k, KEY_LOWEST), KEY_HIGHEST);
+  return __uint_as_float(k ^ ((uint32_t)((int32_t)~k >> 31) | 0x80000000u));
+}
+
+// Maximum over the 64 lanes of a wave (every lane active), in DPP moves as
+// wave_inclusive_scan; lanes shifted in from outside a row keep `v`'s own.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Histogram bins linear in the score over [base, base + span]: non-decreasing
+// in the key; infinities, NaN and keys outside take the end bins.
+struct LinearBins {
+  float base, per_bin;
+  __device__ __forceinline__ int of(uint32_t k) const {
+    return (int)fminf(fmaxf((key_score(k) - base) * per_bin, 0.f), (float)(TK_BINS - 1));
+  }
+  // A key that no key of a bin >= b is below (a hundredth of a bin and one
+  // step of the float against the rounding of either direction).
+  __device__ __forceinline__ uint32_t lower_bound(int b) const {
+    if (b <= 0) return 1u;
+    return score_key(base + ((float)b - 0.01f) / per_bin) - 1u;
+  }
+};
+
+template <int THREADS, int ITEMS, int MODE>
+__global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384 ? 6 : 4) void sparse_topk_row(TopkArgs a) {
+  constexpr int WAVES = THREADS / 64, GROUPS = ITEMS / 4;
+  constexpr int CELLS = GROUPS * WAVES;            // (group, wave) cells, in position order
+  constexpr int PER_LANE = (CELLS + 63) / 64;
+  constexpr int PER_THREAD = TK_ENTRIES / THREADS;  // entries per thread
+  constexpr int SMALL = 64;
+  static_assert(ITEMS % 4 == 0 && (PER_LANE == 1 || WAVES % PER_LANE == 0), "cells of a lane stay in one group");
+  static_assert(PER_THREAD * THREADS == TK_ENTRIES, "entries split evenly");
+  __shared__ RadixLds<false> radix;
+  __shared__ __attribute__((aligned(16))) uint32_t entry_key[TK_ENTRIES];
+  __shared__ __attribute__((aligned(16))) int entry_pos[TK_ENTRIES];
+  __shared__ int request_lds[4];
+  __shared__ uint32_t range_lds[2][WAVES];
+  __shared__ uint32_t small_key[SMALL];
+  __shared__ int small_count;
+  __shared__ uint32_t cells[PER_LANE * 64];
+  const int token = a.first_token + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // ---- the request (thread b holds request b) and the row, in one round trip ----
+  int begin = 0, next = 0, available = 0, residual = 0;
+  const bool early = a.B <= THREADS;  // uniform
+  if (early && tid < a.B) {
+    begin = a.cu[tid];
+    next = a.cu[tid + 1];
+    available = a.seq_cmp[tid];
+    residual = a.residual[tid];
+  }
+  const int64_t first = MODE == TK_SEGMENT ? (int64_t)blockIdx.y * (THREADS * ITEMS) : 0;
+  const int held = MODE == TK_MERGE ? a.segments * a.seg_keep : (int)min<int64_t>(a.C - first, THREADS * ITEMS);
+  const uint32_t* source = MODE == TK_MERGE ? a.seg_key + (size_t)blockIdx.x * held
+                                            : reinterpret_cast<const uint32_t*>(a.scores) + (size_t)token * a.C + first;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(source), (short)0, held * 4, BUFFER_WORD3);
+  auto load_group = [&](int u) {  // past the row: zeros, with no memory traffic
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (u * THREADS + tid) * 16, 0, 0));
+  };
+  uint32_t key[ITEMS];  // the score words, then their keys (0: not a candidate)
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) {
+    const u32x4 x = load_group(u);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) key[4 * u + j] = x[j];
+  }
+  for (int i = 4 * tid; i < 2 * TK_BINS; i += 4 * THREADS)
+    *reinterpret_cast<u32x4*>(&radix.hist[0][0] + i) = u32x4{0u, 0u, 0u, 0u};
+  if (tid == 0) small_count = 0;
+  TokenBounds tb;
+  if (early) {
+    // The last b with cu[b] <= token, request 0 at least (as token_bounds).
+    if (tid < a.B && (begin <= token || tid == 0) && (tid == a.B - 1 || next > token)) {
+      request_lds[0] = begin;
+      request_lds[1] = next;
+      request_lds[2] = available;
+      request_lds[3] = residual;
+    }
+    block_barrier();
+    tb = bounds_of(a, token, request_lds[0], request_lds[1], request_lds[2], request_lds[3]);
+  } else {
+    tb = token_bounds(a, token);
+    block_barrier();
+  }
+  int32_t* out = a.indices + (size_t)token * a.TOPK;
+  uint32_t* seg_key = nullptr;
+  int32_t* seg_pos = nullptr;
+  int cand = tb.cand, take = tb.take;
+  if constexpr (MODE == TK_SEGMENT) {
+    const size_t at = ((size_t)blockIdx.x * a.segments + blockIdx.y) * a.seg_keep;
+    seg_key = a.seg_key + at;
+    seg_pos = a.seg_pos + at;
+    cand = (int)max<int64_t>(0, min<int64_t>(tb.cand - first, held));
+    take = min(take, cand);
+    for (int i = take + tid; i < a.seg_keep; i += THREADS) seg_key[i] = 0u;
+    if (take == 0) return;
+  } else {
+    if (trivial_selection<THREADS>(a, tb, out)) return;
+  }
+  auto position = [&](int i) { return ((i >> 2) * THREADS + tid) * 4 + (i & 3); };  // of key[i]
+  auto emit = [&](int slot, uint32_t k, int p) {
+    if constexpr (MODE == TK_SEGMENT) {
+      seg_key[slot] = k;
+      seg_pos[slot] = (int)first + p;
+    } else if constexpr (MODE == TK_MERGE) {
+      out[slot] = a.seg_pos[(size_t)blockIdx.x * held + p];
+    } else {
+      out[slot] = p;
+    }
+  };
+
+  // ---- 1. bound ------------------------------------------------------------------
+  uint32_t top[GROUPS];  // group maxima, 0 for a group with no candidate
+  uint32_t low = 0xffffffffu, high = 0u;  // finite ones
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) {
+    uint32_t m = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int i = 4 * u + j;
+      if constexpr (MODE != TK_MERGE) key[i] = position(i) < cand ? score_key(__uint_as_float(key[i])) : 0u;
+      key[i] = opaque(key[i]);  // no comparison is kept in scalar registers for the steps below
+      m = max(m, key[i]);
+    }
+    top[u] = m;
+    if (m >= KEY_LOWEST) low = min(low, m);
+    if (m <= KEY_HIGHEST) high = max(high, m);
+  }
+  low = ~wave_max(~low);
+  high = wave_max(high);
+  if (lane == 0) {
+    range_lds[0][wave] = low;
+    range_lds[1][wave] = high;
+  }
+  block_barrier();
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    low = min(low, range_lds[0][w]);
+    high = max(high, range_lds[1][w]);
+  }
+  LinearBins bins;
+  bins.base = key_score(low);
+  const float span = key_score(high) - bins.base;
+  // No finite maximum: low > high, or high below the finite keys.
+  const bool linear = low <= high && high >= KEY_LOWEST && span > 1e-30f && span < 3e38f;
+  bins.per_bin = (TK_BINS - 1) / span;
+  uint32_t bound = 0u;
+  int n = TK_ENTRIES + 1;  // keys that reach the bound
+  uint32_t before[GROUPS];
+  auto scan_cells = [&](auto count) {  // count(u): this thread's (packed) count of group u, at most 4 in each half
+#pragma unroll
+    for (int u = 0; u < GROUPS; ++u) {
+      const int c = count(u), incl = wave_inclusive_scan(c);
+      before[u] = (uint32_t)(incl - c);
+      if (lane == 63) cells[u * WAVES + wave] = (uint32_t)incl;
+    }
+    if (CELLS < 64 && tid >= CELLS && tid < 64) cells[tid] = 0u;
+    block_barrier();
+  };
+  // Sums of the cells before (u, wave) and their total, low and high halves.
+  uint32_t cell[PER_LANE];
+  int lo_excl = 0, hi_excl = 0, lo_total = 0;
+  auto read_cells = [&]() {
+    int lo_sum = 0, hi_sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+      cell[i] = cells[lane * PER_LANE + i];
+      lo_sum += (int)(cell[i] & 0xffffu);
+      hi_sum += (int)(cell[i] >> 16);
+    }
+    const int lo_incl = wave_inclusive_scan(lo_sum);
+    lo_excl = lo_incl - lo_sum;
+    lo_total = __builtin_amdgcn_readlane(lo_incl, 63);
+    hi_excl = wave_inclusive_scan(hi_sum) - hi_sum;
+  };
+  auto cell_base = [&](int u, int& lo, int& hi) {
+    const int at = u * WAVES + wave, owner = at / PER_LANE;  // uniform
+    lo = __builtin_amdgcn_readlane(lo_excl, owner);
+    hi = __builtin_amdgcn_readlane(hi_excl, owner);
+#pragma unroll
+    for (int i = 0; i + 1 < PER_LANE; ++i)
+      if (i < at % PER_LANE) {
+        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cell[i], owner);
+        lo += (int)(c & 0xffffu);
+        hi += (int)(c >> 16);
+      }
+  };
+  if (linear) {  // uniform
+#pragma unroll
+    for (int u = 0; u < GROUPS; ++u)
+      if (top[u] != 0u) atomicAdd(&radix.hist[0][bins.of(top[u])], 1u);
+    block_barrier();
+    if (wave == 0) pick_bin<false, true>(radix, 0, TK_BINS, take, lane);
+    block_barrier();
+    bound = bins.lower_bound(radix.choice[0]);  // fewer groups than `take`: bin 0, every key
+
+    // ---- 2. the keys that reach it, in position order ---------------------------
+    scan_cells([&](int u) {
+      int c = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) c += key[4 * u + j] >= bound ? 1 : 0;
+      return c;
+    });
+    read_cells();
+    n = lo_total;
+  }
+  if (n <= TK_ENTRIES) {  // uniform
+#pragma unroll
+    for (int u = 0; u < GROUPS; ++u) {
+      int slot, unused;
+      cell_base(u, slot, unused);
+      slot += (int)before[u];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t k = opaque(key[4 * u + j]);
+        if (k >= bound) {
+          entry_key[slot] = k;
+          entry_pos[slot] = position(4 * u + j);
+          ++slot;
+        }
+      }
+    }
+    block_barrier();
+
+    // ---- 3. the threshold among them: thread t holds entries PER_THREAD t + e ----
+    uint32_t k[PER_THREAD];
+    int p[PER_THREAD];
+#pragma unroll
+    for (int e = 0; e < PER_THREAD; ++e) {
+      const int i = tid * PER_THREAD + e;
+      k[e] = i < n ? entry_key[i] : 0u;
+      p[e] = entry_pos[i];
+    }
+    bins.base = key_score(max(bound, low));
+    const float rest = key_score(high) - bins.base;
+    bins.per_bin = rest > 1e-30f ? (TK_BINS - 1) / rest : 0.f;  // 0: one bin
+#pragma unroll
+    for (int e = 0; e < PER_THREAD; ++e)
+      if (k[e] != 0u) atomicAdd(&radix.hist[1][bins.of(k[e])], 1u);
+    block_barrier();
+    if (wave == 0)
+      pick_bin<false, true>(radix, 1, TK_BINS, take, lane);
+    else
+      for (int i = tid - 64; i < TK_BINS; i += THREADS - 64) radix.hist[0][i] = 0u;
+    block_barrier();
+    const int bin = radix.choice[0], inside = radix.choice[2];
+    int need = take - radix.choice[1];
+    uint32_t threshold;
+    if (inside <= SMALL) {  // uniform
+#pragma unroll
+      for (int e = 0; e < PER_THREAD; ++e)
+        if (k[e] != 0u && bins.of(k[e]) == bin) small_key[atomicAdd(&small_count, 1)] = k[e];
+      block_barrier();
+      // Every wave ranks them: lane l's key is the threshold when fewer than
+      // `need` keys are larger and, with those equal to it, at least `need`.
+      const uint32_t mine = lane < inside ? small_key[lane] : 0u;
+      int larger = 0, equal = 0;
+      for (int i = 0; i < inside; ++i) {
+        const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
+        larger += other > mine ? 1 : 0;
+        equal += other == mine ? 1 : 0;
+      }
+      const int owner = (int)__builtin_ctzll(__ballot(lane < inside && larger < need && larger + equal >= need));
+      threshold = (uint32_t)__builtin_amdgcn_readlane((int)mine, owner);
+      need -= __builtin_amdgcn_readlane(larger, owner);
+    } else {
+      int parity = 0;
+      threshold = radix_select<THREADS, false>(
+          [&](auto f) {
+#pragma unroll
+            for (int e = 0; e < PER_THREAD; ++e)
+              if (k[e] != 0u && bins.of(k[e]) == bin) f(k[e]);
+          },
+          need, radix, parity, &need);
+    }
+
+    // ---- 4. the taken entries, in order --------------------------------------
+    int c = 0;
+#pragma unroll
+    for (int e = 0; e < PER_THREAD; ++e) c += k[e] > threshold ? 1 : (k[e] == threshold ? 0x10000 : 0);
+    const int incl = wave_inclusive_scan(c);
+    if (lane == 63) cells[wave] = (uint32_t)incl;
+    block_barrier();
+    int above = 0, equal = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      if (w < wave) {
+        above += (int)(cells[w] & 0xffffu);
+        equal += (int)(cells[w] >> 16);
+      }
+    above += (incl - c) & 0xffff;
+    equal += (int)((uint32_t)(incl - c) >> 16);
+#pragma unroll
+    for (int e = 0; e < PER_THREAD; ++e) {
+      const bool gt = k[e] > threshold, eq = k[e] == threshold;
+      const int slot = above + min(equal, need);
+      if ((gt || (eq && equal < need)) && slot < take) emit(slot, k[e], p[e]);
+      above += gt ? 1 : 0;
+      equal += eq ? 1 : 0;
+    }
+    return;
+  }
+
+  // ---- the whole row: radix selection (its keys formed again from memory, a
+  // loop over the registers would be unrolled three times), then the same
+  // counts and slots over the registers.
+  block_barrier();  // every wave has read the cells and the choice
+  for (int i = tid; i < TK_BINS; i += THREADS) radix.hist[0][i] = 0u;
+  block_barrier();
+  int parity = 0, need = 0;
+  const uint32_t threshold = radix_select<THREADS, false>(
+      [&](auto f) {
+        for (int u = 0; u < GROUPS; ++u) {
+          const u32x4 x = load_group(u);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t k = MODE == TK_MERGE                 ? x[j]
+                               : position(4 * u + j) < cand ? score_key(__uint_as_float(x[j]))
+                                                                : 0u;
+            if (k != 0u) f(k);
+          }
+        }
+      },
+      take, radix, parity, &need);
+  scan_cells([&](int u) {
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c += key[4 * u + j] > threshold ? 1 : (key[4 * u + j] == threshold ? 0x10000 : 0);
+    return c;
+  });
+  read_cells();
+#pragma unroll
+  for (int u = 0; u < GROUPS; ++u) {
+    int above, equal;
+    cell_base(u, above, equal);
+    above += (int)(before[u] & 0xffffu);
+    equal += (int)(before[u] >> 16);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t k = opaque(key[4 * u + j]);
+      const bool gt = k > threshold, eq = k == threshold;
+      const int slot = above + min(equal, need);
+      if ((gt || (eq && equal < need)) && slot < take) emit(slot, k, position(4 * u + j));
+      above += gt ? 1 : 0;
+      equal += eq ? 1 : 0;
+    }
+  }
+}
+
 // Streaming form, for rows of any length: every digit re-reads the row, and
 // the output is written chunk by chunk in position order (one scan per chunk
 // of THREADS positions, counting keys equal to the threshold in the high
@@ -647,14 +1072,89 @@ __global__ __launch_bounds__(TK_STREAM_THREADS) void sparse_topk_stream(TopkArgs
 
 using namespace afa;
 
-extern "C" int launch_sparse_topk_indices(void* stream, const float* scores, const int32_t* cu_seqlens_q,
-                                          const int32_t* seqused_cmp_kv, const int32_t* cmp_residual_kv,
-                                          int32_t* cmp_sparse_indices, const SparseTopkParams* params) {
+// Form of a call. ROW and SPLIT are the register forms (sparse_topk_row), for
+// calls of few enough tokens that a row's chain of steps, not the scores'
+// bytes, sets the time; FILTER and STREAM the streaming ones.
+enum TopkForm { TK_FORM_ROW, TK_FORM_SPLIT, TK_FORM_FILTER, TK_FORM_STREAM };
+struct TopkPlan {
+  TopkForm form;
+  int threads, items;  // ROW
+  int segments, keep;  // SPLIT: segments of TK_SEGMENT_SIZE positions, entries kept of each
+  int64_t tokens;      // SPLIT: tokens per pair of launches
+};
+constexpr int TK_SEGMENT_ITEMS = 16;
+constexpr int64_t TK_SEGMENT_SIZE = 1024 * TK_SEGMENT_ITEMS;
+constexpr int64_t TK_MERGE_MAX = 1024 * 32;  // entries of all segments of a row
+constexpr int64_t TK_SPLIT_WORKGROUPS = 2048;
+constexpr int64_t TK_SPLIT_BYTES = int64_t(64) << 20;  // workspace of a call, at most (one token at least)
+
+// Whether the keys of a row of C that reach sparse_topk_row's bound are
+// expected to fit its entries: with a fraction f = TOPK / (C / 4) of the groups
+// above the threshold, 1 - (1 - f)^(1/4) of the keys are. Rows that do not fit
+// give the same result through a radix selection, later.
+static bool row_fits(int64_t C, int64_t topk) {
+  if (C <= TK_ENTRIES) return true;
+  const double f = 4.0 * (double)topk / (double)C;
+  return f < 1.0 && (double)C * (1.0 - std::sqrt(std::sqrt(1.0 - f))) <= 0.93 * TK_ENTRIES;
+}
+
+// Lines of the form, measured either side (us, register form / streaming form,
+// TOPK 512 unless stated): rows of 8K
+// 2000 24.6 / 25.7, 4096 45.2 / 45.0; of 16K 6000 103.6 / 109.9, 8192 135.6 /
+// 134.5; of 16.4K 1000 39.2 / 44.4, 2000 72.0 / 54.1 (a 32K row's registers half
+// empty); of 30K 1000 48.8 / 77.0. Split rows of 128K (8 segments): 64 22.5 /
+// 33.3, 600 118 / 107; of 256K 128 (2048 segments) 56.9 / 90; rows of 64K 6 21.7 /
+// 20.1, 384 47.0 / 32.9. 1961 rows of 2.7K with TOPK 1024, which do not fit the
+// entries, 31.1 / 29.6.
+static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
+  TopkPlan plan{};
+  const int64_t C = p->C, T = p->T;
+  const bool fits = row_fits(C, p->TOPK);
+  const int64_t most = C <= 8192 ? 2048 : C <= 16384 ? 6144 : 1024;
+  if (C <= 32768 && T <= most && fits) {
+    plan.form = TK_FORM_ROW;
+    // One 1024-thread workgroup per CU while every token gets a CU of its own,
+    // smaller workgroups, more of which share a CU, beyond.
+    plan.threads = T <= 256 ? 1024 : 512;
+    plan.items = 4;
+    while ((int64_t)plan.threads * plan.items < C) plan.items *= 2;
+    if (plan.threads == 512) plan.items = std::max(plan.items, 8);
+    return plan;
+  }
+  const int64_t segments = (C + TK_SEGMENT_SIZE - 1) / TK_SEGMENT_SIZE;
+  const int64_t keep = (std::min<int64_t>(p->TOPK, TK_SEGMENT_SIZE) + 3) / 4 * 4;
+  if (with_workspace && C > 65536 && segments * keep <= TK_MERGE_MAX &&
+      (C > TK_FILTER_MAX_C || T * segments <= TK_SPLIT_WORKGROUPS)) {
+    plan.form = TK_FORM_SPLIT;
+    plan.segments = (int)segments;
+    plan.keep = (int)keep;
+    plan.tokens = std::min(T, std::max<int64_t>(1, TK_SPLIT_BYTES / (segments * keep * 8)));
+    return plan;
+  }
+  plan.form = C <= TK_FILTER_MAX_C ? TK_FORM_FILTER : TK_FORM_STREAM;
+  return plan;
+}
+
+static uint64_t topk_split_bytes(const SparseTopkParams* p, const TopkPlan& plan) {
+  return plan.form == TK_FORM_SPLIT ? (uint64_t)plan.tokens * plan.segments * plan.keep * 8 : 0;
+}
+
+static int check_topk(const SparseTopkParams* params) {
   if (!params) return AFA_E_NULL;
   if (params->B <= 0 || params->T <= 0 || params->TOPK <= 0 || params->C <= 0) return AFA_E_SHAPE;
   if (params->RATIO != 1 && params->RATIO != 2) return AFA_E_SHAPE;
   if (params->C > 0x7fffffffLL) return AFA_E_SHAPE;
-  if (!scores || !cu_seqlens_q || !seqused_cmp_kv || !cmp_residual_kv || !cmp_sparse_indices) return AFA_E_NULL;
+  return AFA_OK;
+}
+
+template <int THREADS, int ITEMS, int MODE>
+static void launch_row(const TopkArgs& a, dim3 grid, hipStream_t s) {
+  hipLaunchKernelGGL((sparse_topk_row<THREADS, ITEMS, MODE>), grid, dim3(THREADS), 0, s, a);
+}
+
+static int launch_topk(hipStream_t s, const float* scores, const int32_t* cu_seqlens_q, const int32_t* seqused_cmp_kv,
+                       const int32_t* cmp_residual_kv, int32_t* cmp_sparse_indices, void* workspace,
+                       const SparseTopkParams* params, const TopkPlan& plan) {
   TopkArgs a;
   a.scores = scores;
   a.cu = cu_seqlens_q;
@@ -666,32 +1166,104 @@ extern "C" int launch_sparse_topk_indices(void* stream, const float* scores, con
   a.T = params->T;
   a.TOPK = params->TOPK;
   a.RATIO = params->RATIO;
-  const bool vec = (params->C % 4 == 0) && (reinterpret_cast<uintptr_t>(scores) % 16 == 0);
-  hipStream_t s = (hipStream_t)stream;
+  a.cap = a.words = a.first_token = a.segments = a.seg_keep = 0;
+  a.seg_key = nullptr;
+  a.seg_pos = nullptr;
   const dim3 grid((unsigned)a.T);
-  a.words = (int32_t)((a.C + 31) / 32);
-  // Buffer: rows up to 32K positions (16-bit positions) hold 2 TOPK entries,
-  // between 1024 and 8192, so that little of a CU's LDS is spent on it at the
-  // usual TOPK; longer rows hold TK_WIDE_CAP.
-  a.cap = a.C <= 32768 ? (int32_t)std::min<int64_t>(8192, std::max<int64_t>(1024, ((int64_t)a.TOPK * 2 + 255) / 256 * 256))
-                       : TK_WIDE_CAP;
-  if (a.C <= TK_FILTER_MAX_C) {
-    const size_t dynamic_bytes = 2 * 4 * (size_t)a.words + (a.C <= 32768 ? (size_t)a.cap * 6 : 0);
-    // Rows up to 32K positions: 256 threads, more workgroups per CU; longer
-    // rows: 1024 threads, more loads in flight per row.
-    if (a.C <= 32768) {
-      if (vec)
-        hipLaunchKernelGGL((sparse_topk_filter<256, true>), grid, dim3(256), dynamic_bytes, s, a);
-      else
-        hipLaunchKernelGGL((sparse_topk_filter<256, false>), grid, dim3(256), dynamic_bytes, s, a);
-    } else {
-      if (vec)
-        hipLaunchKernelGGL((sparse_topk_filter<1024, true>), grid, dim3(1024), dynamic_bytes, s, a);
-      else
-        hipLaunchKernelGGL((sparse_topk_filter<1024, false>), grid, dim3(1024), dynamic_bytes, s, a);
+  switch (plan.form) {
+    case TK_FORM_ROW:
+      switch (plan.threads * 100 + plan.items) {
+        case 102404: launch_row<1024, 4, TK_ROW>(a, grid, s); break;
+        case 102408: launch_row<1024, 8, TK_ROW>(a, grid, s); break;
+        case 102416: launch_row<1024, 16, TK_ROW>(a, grid, s); break;
+        case 102432: launch_row<1024, 32, TK_ROW>(a, grid, s); break;
+        case 51208: launch_row<512, 8, TK_ROW>(a, grid, s); break;
+        case 51216: launch_row<512, 16, TK_ROW>(a, grid, s); break;
+        case 51232: launch_row<512, 32, TK_ROW>(a, grid, s); break;
+        default: launch_row<512, 64, TK_ROW>(a, grid, s); break;
+      }
+      break;
+    case TK_FORM_SPLIT: {
+      a.segments = plan.segments;
+      a.seg_keep = plan.keep;
+      a.seg_key = (uint32_t*)workspace;
+      a.seg_pos = (int32_t*)workspace + (size_t)plan.tokens * a.segments * a.seg_keep;
+      const int entries = a.segments * a.seg_keep;
+      for (int64_t t = 0; t < a.T; t += plan.tokens) {
+        a.first_token = (int32_t)t;
+        const unsigned n = (unsigned)std::min<int64_t>(plan.tokens, a.T - t);
+        launch_row<1024, TK_SEGMENT_ITEMS, TK_SEGMENT>(a, dim3(n, (unsigned)a.segments), s);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+        if (entries <= 1024 * 4)
+          launch_row<1024, 4, TK_MERGE>(a, dim3(n), s);
+        else if (entries <= 1024 * 16)
+          launch_row<1024, 16, TK_MERGE>(a, dim3(n), s);
+        else
+          launch_row<1024, 32, TK_MERGE>(a, dim3(n), s);
+        const hipError_t m = hipGetLastError();
+        if (m != hipSuccess) return (int)m;
+      }
+      break;
     }
-  } else {
-    hipLaunchKernelGGL(sparse_topk_stream, grid, dim3(TK_STREAM_THREADS), 0, s, a);
+    case TK_FORM_FILTER: {
+      const bool vec = (params->C % 4 == 0) && (reinterpret_cast<uintptr_t>(scores) % 16 == 0);
+      a.words = (int32_t)((a.C + 31) / 32);
+      // Buffer: rows up to 32K positions (16-bit positions) hold 2 TOPK entries,
+      // between 1024 and 8192, so that little of a CU's LDS is spent on it at the
+      // usual TOPK; longer rows hold TK_WIDE_CAP.
+      a.cap = a.C <= 32768
+                  ? (int32_t)std::min<int64_t>(8192, std::max<int64_t>(1024, ((int64_t)a.TOPK * 2 + 255) / 256 * 256))
+                  : TK_WIDE_CAP;
+      const size_t dynamic_bytes = 2 * 4 * (size_t)a.words + (a.C <= 32768 ? (size_t)a.cap * 6 : 0);
+      // Rows up to 32K positions: 256 threads, more workgroups per CU; longer
+      // rows: 1024 threads, more loads in flight per row.
+      if (a.C <= 32768) {
+        if (vec)
+          hipLaunchKernelGGL((sparse_topk_filter<256, true>), grid, dim3(256), dynamic_bytes, s, a);
+        else
+          hipLaunchKernelGGL((sparse_topk_filter<256, false>), grid, dim3(256), dynamic_bytes, s, a);
+      } else {
+        if (vec)
+          hipLaunchKernelGGL((sparse_topk_filter<1024, true>), grid, dim3(1024), dynamic_bytes, s, a);
+        else
+          hipLaunchKernelGGL((sparse_topk_filter<1024, false>), grid, dim3(1024), dynamic_bytes, s, a);
+      }
+      break;
+    }
+    default: hipLaunchKernelGGL(sparse_topk_stream, grid, dim3(TK_STREAM_THREADS), 0, s, a); break;
   }
   return (int)hipGetLastError();
+}
+
+extern "C" int launch_sparse_topk_indices(void* stream, const float* scores, const int32_t* cu_seqlens_q,
+                                          const int32_t* seqused_cmp_kv, const int32_t* cmp_residual_kv,
+                                          int32_t* cmp_sparse_indices, const SparseTopkParams* params) {
+  const int status = check_topk(params);
+  if (status) return status;
+  if (!scores || !cu_seqlens_q || !seqused_cmp_kv || !cmp_residual_kv || !cmp_sparse_indices) return AFA_E_NULL;
+  return launch_topk((hipStream_t)stream, scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, cmp_sparse_indices,
+                     nullptr, params, choose_topk(params, false));
+}
+
+extern "C" int workspace_size_sparse_topk_indices_split(uint64_t* bytes, const SparseTopkParams* params) {
+  if (!bytes) return -1;
+  const int status = check_topk(params);
+  if (status) return status;
+  *bytes = topk_split_bytes(params, choose_topk(params, true));
+  return AFA_OK;
+}
+
+extern "C" int launch_sparse_topk_indices_split(void* stream, const float* scores, const int32_t* cu_seqlens_q,
+                                                const int32_t* seqused_cmp_kv, const int32_t* cmp_residual_kv,
+                                                int32_t* cmp_sparse_indices, void* workspace, uint64_t workspace_bytes,
+                                                const SparseTopkParams* params) {
+  const int status = check_topk(params);
+  if (status) return status;
+  if (!scores || !cu_seqlens_q || !seqused_cmp_kv || !cmp_residual_kv || !cmp_sparse_indices) return AFA_E_NULL;
+  const TopkPlan plan = choose_topk(params, true);
+  const uint64_t need = topk_split_bytes(params, plan);
+  if (need > 0 && (!workspace || workspace_bytes < need)) return AFA_E_WORKSPACE;
+  return launch_topk((hipStream_t)stream, scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, cmp_sparse_indices,
+                     workspace, params, plan);
 }

@@ -22,6 +22,7 @@ framework can trace the indexer -> top-k -> ``sparse_flash_mla`` chain.
 from __future__ import annotations
 
 import ctypes as ct
+import functools
 
 import torch
 
@@ -37,6 +38,16 @@ class SparseTopkParams(ct.Structure):
         ("RATIO", ct.c_int32),
         ("C", ct.c_int64),
     ]
+
+
+@functools.lru_cache(maxsize=64)
+def _launch_state(lib, B, T, TOPK, RATIO, C):
+    """Launcher parameters and workspace bytes of one set of sizes (neither changes afterwards)."""
+    params = SparseTopkParams(B, T, TOPK, RATIO, C)
+    nbytes = ct.c_uint64(0)
+    _native.check(lib.workspace_size_sparse_topk_indices_split(ct.byref(nbytes), ct.byref(params)),
+                  "workspace_size_sparse_topk_indices_split")
+    return ct.pointer(params), nbytes.value
 
 
 def sparse_topk_indices(scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, TOPK=512, RATIO=2, out=None):
@@ -71,17 +82,22 @@ def sparse_topk_indices(scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, T
             ("cmp_sparse_indices", out, True),
         ]
     )
-    params = SparseTopkParams(b, t, TOPK, RATIO, c)
-    status = _native.library().launch_sparse_topk_indices(
+    lib = _native.library()
+    params, nbytes = _launch_state(lib, b, t, TOPK, RATIO, c)
+    # Entries of split rows; the caching allocator keeps the block for this stream.
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    status = lib.launch_sparse_topk_indices_split(
         stream_handle(device),
         scores.data_ptr(),
         cu_seqlens_q.data_ptr(),
         seqused_cmp_kv.data_ptr(),
         cmp_residual_kv.data_ptr(),
         out.data_ptr(),
-        ct.byref(params),
+        None if workspace is None else workspace.data_ptr(),
+        nbytes,
+        params,
     )
-    _native.check(status, "launch_sparse_topk_indices")
+    _native.check(status, "launch_sparse_topk_indices_split")
     return out
 
 

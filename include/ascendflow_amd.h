@@ -277,6 +277,18 @@ int launch_sparse_topk_indices(void* stream, const float* scores, const int32_t*
                                const int32_t* seqused_cmp_kv, const int32_t* cmp_residual_kv,
                                int32_t* cmp_sparse_indices, const SparseTopkParams* params);
 
+/* The same selection with a workspace for few long rows (decode at long
+ * contexts): each row's segments are selected by workgroups of their own, whose
+ * entries a second launch merges. workspace_size_sparse_topk_indices_split gives
+ * the bytes a call needs (0 where one launch does it, and then `workspace` may
+ * be NULL); the launcher returns AFA_E_WORKSPACE, before any launch, for less.
+ * Results are those of launch_sparse_topk_indices, value for value. */
+int workspace_size_sparse_topk_indices_split(uint64_t* bytes, const SparseTopkParams* params);
+int launch_sparse_topk_indices_split(void* stream, const float* scores, const int32_t* cu_seqlens_q,
+                                     const int32_t* seqused_cmp_kv, const int32_t* cmp_residual_kv,
+                                     int32_t* cmp_sparse_indices, void* workspace, uint64_t workspace_bytes,
+                                     const SparseTopkParams* params);
+
 /* Measurement helpers (no reference kernel; the reference sweeps a >= 4x L2
  * buffer before each timed launch, benchmarks/cache.py:13-92 and
  * benchmarks/cache_sweep.py:15-32). Reads `bytes` of `buffer` through the
