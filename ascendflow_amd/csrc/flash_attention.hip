@@ -739,98 +739,128 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaSplitArgs args) {
   *(x4*)((scalar*)a.o + row * 128 + 4 * u) = v;
 }
 
-// Teaching attention: one workgroup per (head, 64 query rows), 4 waves of 16
-// queries; the whole 128-key tile is resident, so the softmax is exact and P
-// is normalised before its f16 cast (simple.py:25-41).
-__global__ __launch_bounds__(256) void simple_attention_kernel(const _Float16* Qp,
-                                                               const _Float16* Kp,
-                                                               const _Float16* Vp, _Float16* Op,
-                                                               int64_t S) {
+// Teaching attention: the whole 128-key tile of a head is resident in LDS, so
+// the softmax is exact and P is normalised before its f16 cast
+// (simple.py:25-41). A workgroup of four waves takes `steps` consecutive tiles
+// of 64 query rows of one head, 16 rows per wave. Bound by HBM (Q read, O
+// written once); what the split saves is the rest: K and V are loaded once per
+// `steps` tiles instead of once per tile, the next tile's Q loads run under
+// this tile's work, and O leaves through a wave-private LDS stage in whole
+// 256-byte rows (straight from the accumulators a store instruction writes 16
+// pieces of 32 bytes). Two workgroups share a CU (80 KiB of LDS each). Two row
+// tiles per wave, which read each fragment for twice the MFMAs, measured the
+// same. Measured call, one tile per workgroup -> this: H32 S8192 67.1 -> 36.1
+// us (3.8 TB/s), H64 S8192 132.8 -> 61.0 (4.4 TB/s), H64 S2048 29.1 -> 17.6.
+__global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16* Qp, const _Float16* Kp,
+                                                                  const _Float16* Vp, _Float16* Op, int64_t S,
+                                                                  int32_t groups, int32_t steps) {
   typedef B16<DT_F16> ops;
-  constexpr int D = 128, SK = 128, ROW_BYTES = D * 2, KT = SK / 16;
+  constexpr int D = 128, SK = 128, ROW_BYTES = D * 2, KT = SK / 16, ROWS = 16;
   __shared__ __attribute__((aligned(16))) uint8_t k_lds[SK * ROW_BYTES];
   __shared__ __attribute__((aligned(16))) uint8_t v_lds[SK * ROW_BYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t o_lds[4][16 * ROW_BYTES];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int g = lane >> 4, i16 = lane & 15;
-  const int64_t tiles = S / 64;
-  const int64_t head = blockIdx.x / tiles, tile = blockIdx.x % tiles;
+  const uint32_t logical = xcd_contiguous(blockIdx.x, gridDim.x);  // a head's groups share its K and V in one L2
+  const int64_t head = logical / (uint32_t)groups, group = logical % (uint32_t)groups;
   const _Float16* Q = Qp + head * S * D;
   const _Float16* K = Kp + head * SK * D;
   const _Float16* V = Vp + head * SK * D;
   _Float16* O = Op + head * S * D;
+  // This wave's first row of step s (S is a multiple of 64: a wave's rows are all in or all out).
+  auto first_row = [&](int s) { return ((group * steps + s) * 4 + wave) * ROWS; };
 
+  f16x8 qf[D / 32];
+  auto load_q = [&](int s) {
+    const int64_t row = first_row(s);
+    if (row < S) {
+#pragma unroll
+      for (int j = 0; j < D / 32; ++j) qf[j] = *(const f16x8*)(Q + (row + i16) * D + 32 * j + 8 * g);
+    }
+  };
+  load_q(0);
   for (int flat = tid; flat < SK * (D / 8); flat += 256) {
     const int r = flat / (D / 8), u = flat % (D / 8);
     const int off = r * ROW_BYTES + (swz(r, u) << 4);
     *(u32x4*)(&k_lds[off]) = *(const u32x4*)(K + r * D + u * 8);
     *(u32x4*)(&v_lds[off]) = *(const u32x4*)(V + r * D + u * 8);
   }
-  const int64_t query = tile * 64 + wave * 16 + i16;
-  f16x8 qf[D / 32];
-#pragma unroll
-  for (int j = 0; j < D / 32; ++j) qf[j] = *(const f16x8*)(Q + query * D + 32 * j + 8 * g);
   __syncthreads();
 
   const int ra = sigma(i16);
-  f32x4 s[KT];
-#pragma unroll
-  for (int t = 0; t < KT; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < D / 32; ++j) {
-    const int u = 4 * j + g;
-#pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      const int row = 16 * t + ra;
-      const f16x8 kf = *(const f16x8*)(k_lds + row * ROW_BYTES + (swz(row, u) << 4));
-      s[t] = ops::mfma(kf, qf[j], s[t]);
-    }
-  }
-  const float scale_log2 = 0.08838834764831845f * FA_LOG2E;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int t = 0; t < KT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[t][i] *= scale_log2;
-      mx = fmaxf(mx, s[t][i]);
-    }
-  mx = max_over_lane_groups(mx);
-  float sum = 0.f;
-#pragma unroll
-  for (int t = 0; t < KT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      s[t][i] = fast_exp2(s[t][i] - mx);
-      sum += s[t][i];
-    }
-  const float inv = 1.0f / sum_over_lane_groups(sum);
-  f16x8 pf[SK / 32];
-#pragma unroll
-  for (int t = 0; t < KT; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pf[t >> 1][(t & 1) * 4 + i] = (_Float16)(s[t][i] * inv);
-
   const int rt = sigma(4 * g + (i16 >> 2));
   const int tr_half = (i16 & 1) * 8, tr_unit = (i16 & 3) >> 1;
-  _Float16* orow = O + query * D + 4 * g;
+  const float scale_log2 = 0.08838834764831845f * FA_LOG2E;
+  for (int step = 0; step < steps; ++step) {
+    const int64_t row0 = first_row(step);
+    if (row0 >= S) break;
+    f32x4 s[KT];
 #pragma unroll
-  for (int t = 0; t < D / 16; ++t) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    const int u = 2 * t + tr_unit;
+    for (int t = 0; t < KT; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < SK / 32; ++ks) {
-      const int r0 = 32 * ks + rt, r1 = 32 * ks + 16 + rt;
-      const f16x4 lo = ops::read_tr(
-          (const AFA_LDS void*)(v_lds + r0 * ROW_BYTES + (swz(r0, u) << 4) + tr_half));
-      const f16x4 hi = ops::read_tr(
-          (const AFA_LDS void*)(v_lds + r1 * ROW_BYTES + (swz(r1, u) << 4) + tr_half));
-      const f16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      acc = ops::mfma(vf, pf[ks], acc);
+    for (int j = 0; j < D / 32; ++j) {
+      const int u = 4 * j + g;
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+        const int row = 16 * t + ra;
+        const f16x8 kf = *(const f16x8*)(k_lds + row * ROW_BYTES + (swz(row, u) << 4));
+        s[t] = ops::mfma(kf, qf[j], s[t]);
+      }
     }
-    f16x4 v;
+    if (step + 1 < steps) load_q(step + 1);  // lands during the softmax and PV
+    float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = (_Float16)acc[i];
-    *(f16x4*)(orow + 16 * t) = v;
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[t][i] *= scale_log2;
+        mx = fmaxf(mx, s[t][i]);
+      }
+    mx = max_over_lane_groups(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[t][i] = fast_exp2(s[t][i] - mx);
+        sum += s[t][i];
+      }
+    const float inv = 1.0f / sum_over_lane_groups(sum);
+    f16x8 pf[SK / 32];
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pf[t >> 1][(t & 1) * 4 + i] = (_Float16)(s[t][i] * inv);
+    f32x4 acc[D / 16];
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int u = 2 * t + tr_unit;
+#pragma unroll
+      for (int ks = 0; ks < SK / 32; ++ks) {
+        const int r0 = 32 * ks + rt, r1 = 32 * ks + 16 + rt;
+        const f16x4 lo = ops::read_tr((const AFA_LDS void*)(v_lds + r0 * ROW_BYTES + (swz(r0, u) << 4) + tr_half));
+        const f16x4 hi = ops::read_tr((const AFA_LDS void*)(v_lds + r1 * ROW_BYTES + (swz(r1, u) << 4) + tr_half));
+        const f16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        acc[t] = ops::mfma(vf, pf[ks], acc[t]);
+      }
+    }
+    // This lane holds features 16t + 4g + 0..3 of row i16: staged as 16-byte
+    // unit u of row r at u ^ r, read back four whole rows per access. Only this
+    // wave touches the stage, and its LDS operations complete in order.
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      f16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (_Float16)acc[t][i];
+      *(f16x4*)(&o_lds[wave][i16 * ROW_BYTES + (((2 * t + (g >> 1)) ^ i16) << 4) + (g & 1) * 8]) = v;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = 4 * q + g;  // lane 16g + i16 takes unit i16 of it
+      const u32x4 v = *(const u32x4*)(&o_lds[wave][r * ROW_BYTES + ((i16 ^ r) << 4)]);
+      *(u32x4*)(O + (row0 + r) * D + 8 * i16) = v;
+    }
   }
 }
 
@@ -1030,9 +1060,22 @@ extern "C" int launch_simple_attention(void* stream, const void* Q, const void* 
   (void)workspace;
   if (!Q || !K || !V || !O) return AFA_E_NULL;
   if (S <= 0 || S % 64 || H <= 0 || (S / 64) * H > 0x7fffffffLL) return AFA_E_SHAPE;
-  hipLaunchKernelGGL(simple_attention_kernel, dim3((unsigned)((S / 64) * H)), dim3(256), 0,
-                     (hipStream_t)stream, (const _Float16*)Q, (const _Float16*)K,
-                     (const _Float16*)V, (_Float16*)O, S);
+  // Tiles per workgroup that take the fewest rounds of two workgroups per CU,
+  // each as long as its tiles and about one more for K and V (H36 S6912: 6 tiles
+  // 33.1 us, 3 tiles, whose 1.3 rounds end with an idle GPU, 38.4).
+  const int64_t slots = 2 * FA_CUS, tiles = S / 64;
+  int64_t steps = 1, best = INT64_MAX;
+  for (int64_t k = 1; k <= std::min<int64_t>(tiles, 16); ++k) {
+    const int64_t cost = (((tiles + k - 1) / k * H + slots - 1) / slots) * (k + 1);
+    if (cost < best) {
+      best = cost;
+      steps = k;
+    }
+  }
+  const int64_t groups = (tiles + steps - 1) / steps;
+  hipLaunchKernelGGL(simple_attention_kernel, dim3((unsigned)(groups * H)), dim3(256), 0, (hipStream_t)stream,
+                     (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, S, (int32_t)groups,
+                     (int32_t)steps);
   return (int)hipGetLastError();
 }
 
