@@ -13,8 +13,13 @@ import torch
 DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16}
 
 
+_STORAGE_NAMES = {"bf16": "bf16", "f16": "f16", torch.bfloat16: "bf16", torch.float16: "f16"}
+
+
 def storage_dtype(value) -> str:
     """Normalise a DTYPE constexpr ("bf16"/"f16", torch dtype or an object named so)."""
+    if isinstance(value, (str, torch.dtype)) and value in _STORAGE_NAMES:
+        return _STORAGE_NAMES[value]
     if isinstance(value, torch.dtype):
         for name, dt in DTYPES.items():
             if dt == value:
@@ -57,6 +62,44 @@ def check_disjoint(named):
             if j != i and a0 < b1 and b0 < a1:
                 first, second = (a, b) if i < j else (b, a)
                 raise ValueError(f"external tensors {first} and {second} overlap")
+
+
+class Operand:
+    """Shape, dtype and bytes that a call of given sizes expects of one tensor."""
+
+    __slots__ = ("name", "shape", "dtype", "nbytes")
+
+    def __init__(self, name, shape, dtype):
+        self.name = name
+        self.shape = torch.Size(shape)
+        self.dtype = dtype
+        self.nbytes = self.shape.numel() * dtype.itemsize
+
+
+def operand_pointers(operands, tensors, written):
+    """(device index, data pointers) of a call's tensors after the checks of
+    ``check_tensor`` and, for the operand at index ``written``, of
+    ``check_disjoint``, each tensor looked at once (an eager call of a few
+    microseconds on the GPU is otherwise bound by its checks); a failure is
+    reported by those two."""
+    device = tensors[0].get_device() if isinstance(tensors[0], torch.Tensor) and tensors[0].is_cuda else -1
+    pointers = []
+    for o, t in zip(operands, tensors):
+        if (device < 0 or not isinstance(t, torch.Tensor) or t.dtype is not o.dtype or t.shape != o.shape
+                or t.get_device() != device or not t.is_contiguous()):
+            check_tensor(o.name, t, o.shape, o.dtype, tensors[0].device if pointers else None)
+        pointers.append(t.data_ptr())
+    start = pointers[written]
+    end = start + operands[written].nbytes
+    for i, p in enumerate(pointers):
+        if p < end and start < p + operands[i].nbytes and i != written:
+            check_disjoint([(o.name, t, i == written) for i, (o, t) in enumerate(zip(operands, tensors))])
+    return device, pointers
+
+
+def raw_stream(device_index) -> int:
+    """Handle of the current stream of a device."""
+    return torch._C._cuda_getCurrentRawStream(device_index)
 
 
 def stream_handle(device) -> int:

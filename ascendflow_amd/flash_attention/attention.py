@@ -18,7 +18,7 @@ import functools
 import torch
 
 from .. import _native
-from .._tensors import DTYPES, check_disjoint, check_tensor, require, storage_dtype, stream_handle
+from .._tensors import DTYPES, Operand, operand_pointers, raw_stream, require, storage_dtype
 
 
 def causal_policy(sq, sk):
@@ -31,16 +31,37 @@ def causal_policy(sq, sk):
     return {"kv_tile": 1024, "vector_rows": 8}
 
 
+class _Call:
+    """Checked sizes of a call: its operands, launcher parameters and workspace bytes (none changes afterwards)."""
+
+    __slots__ = ("Sq", "Sk", "operands", "params", "nbytes", "launch")
+
+
 @functools.lru_cache(maxsize=64)
-def _launch_state(lib, B, HQ, HKV, D, dtype, causal, scale, Sq, Sk):
-    """Launcher parameters and workspace bytes of one set of sizes (neither changes afterwards)."""
+def _call(lib, Sq, Sk, B, HQ, HKV, D, BQ, BM, BK, CK, VR, GROUPS, dtype, SCALE, causal):
+    require(Sq >= 1 and Sk >= 1, "Sq and Sk must be >= 1")
+    require(B > 0 and HQ > 0 and HKV > 0, "positive batch and head counts")
+    require(HQ % HKV == 0, "query heads must be divisible by KV heads")
+    require(VR > 0 and BQ % (2 * VR) == 0, "query tile must cover complete rows on both AIVs")
+    require(BM > 0 and BQ % BM == 0 and BQ <= 2 * BM, "query tile must fit the accumulator planes")
+    require(CK > 0 and BK % CK == 0 and CK == D, "KV tile must contain complete CK == D chunks")
+    require(GROUPS > 0 and SCALE > 0, "positive worker count and scale")
+    require(D == 128, "gfx950 kernel supports D = 128")
+    b16 = DTYPES[dtype]
+    call = _Call()
+    call.Sq, call.Sk = Sq, Sk
+    call.operands = (Operand("Q", (B, HQ, Sq, D), b16), Operand("K", (B, HKV, Sk, D), b16),
+                     Operand("V", (B, HKV, Sk, D), b16), Operand("O", (B, HQ, Sq, D), b16))
     params = _native.FaParams(
-        B=B, HQ=HQ, HKV=HKV, D=D, dtype=_native.AFA_DTYPE[dtype], causal=int(causal), scale=scale, reserved=0
+        B=B, HQ=HQ, HKV=HKV, D=D, dtype=_native.AFA_DTYPE[dtype], causal=int(causal), scale=SCALE, reserved=0
     )
     nbytes = ct.c_uint64(0)
     _native.check(lib.workspace_size_attention_target_split(ct.byref(nbytes), Sq, Sk, ct.byref(params)),
                   "workspace_size_attention_target_split")
-    return ct.pointer(params), nbytes.value
+    call.params = ct.pointer(params)
+    call.nbytes = nbytes.value
+    call.launch = lib.launch_attention_target_split
+    return call
 
 
 def attention_target(
@@ -65,29 +86,15 @@ def attention_target(
     CAUSAL=False,
 ):
     """FA forward: O[B,HQ,Sq,D] = softmax(Q K^T * SCALE [+ causal mask]) V."""
-    dtype = storage_dtype(DTYPE)
-    Sq, Sk = int(Sq), int(Sk)
-    require(Sq >= 1 and Sk >= 1, "Sq and Sk must be >= 1")
-    require(B > 0 and HQ > 0 and HKV > 0, "positive batch and head counts")
-    require(HQ % HKV == 0, "query heads must be divisible by KV heads")
-    require(VR > 0 and BQ % (2 * VR) == 0, "query tile must cover complete rows on both AIVs")
-    require(BM > 0 and BQ % BM == 0 and BQ <= 2 * BM, "query tile must fit the accumulator planes")
-    require(CK > 0 and BK % CK == 0 and CK == D, "KV tile must contain complete CK == D chunks")
-    require(GROUPS > 0 and SCALE > 0, "positive worker count and scale")
-    require(D == 128, "gfx950 kernel supports D = 128")
-    b16 = DTYPES[dtype]
-    check_tensor("Q", Q, (B, HQ, Sq, D), b16)
-    check_tensor("K", K, (B, HKV, Sk, D), b16, Q.device)
-    check_tensor("V", V, (B, HKV, Sk, D), b16, Q.device)
-    check_tensor("O", O, (B, HQ, Sq, D), b16, Q.device)
-    check_disjoint([("Q", Q, False), ("K", K, False), ("V", V, False), ("O", O, True)])
-    lib = _native.library()
-    params, nbytes = _launch_state(lib, B, HQ, HKV, D, dtype, bool(CAUSAL), SCALE, Sq, Sk)
-    # Partial results of split keys; the caching allocator keeps the block for this stream.
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=Q.device) if nbytes else None
-    status = lib.launch_attention_target_split(
-        stream_handle(Q.device), Q.data_ptr(), K.data_ptr(), V.data_ptr(), O.data_ptr(),
-        None if workspace is None else workspace.data_ptr(), nbytes, Sq, Sk, params
-    )
-    _native.check(status, "launch_attention_target_split")
+    call = _call(_native.library(), int(Sq), int(Sk), B, HQ, HKV, D, BQ, BM, BK, CK, VR, GROUPS,
+                 storage_dtype(DTYPE), SCALE, bool(CAUSAL))
+    device, (q, k, v, o) = operand_pointers(call.operands, (Q, K, V, O), 3)
+    workspace = None
+    if call.nbytes:
+        # Partial results of split keys; the caching allocator keeps the block for this stream.
+        scratch = torch.empty(call.nbytes, dtype=torch.uint8, device=Q.device)
+        workspace = scratch.data_ptr()
+    status = call.launch(raw_stream(device), q, k, v, o, workspace, call.nbytes, call.Sq, call.Sk, call.params)
+    if status:
+        _native.check(status, "launch_attention_target_split")
     return O

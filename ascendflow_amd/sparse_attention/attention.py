@@ -263,7 +263,7 @@ def _prepare(
         require(workspace.numel() >= b.nbytes, f"workspace holds {workspace.numel()} bytes, needs {b.nbytes}")
         extra += (("workspace", workspace),)
     elif b.nbytes:
-        if torch.cuda.is_current_stream_capturing():
+        if torch._C._cuda_isCurrentStreamCapturing():
             workspace = torch.empty(b.nbytes, dtype=torch.uint8, device=b.device)
         else:
             if b.workspace is None:

@@ -27,7 +27,7 @@ import functools
 import torch
 
 from .. import _native
-from .._tensors import check_disjoint, check_tensor, require, stream_handle
+from .._tensors import Operand, operand_pointers, raw_stream, require
 
 
 class SparseTopkParams(ct.Structure):
@@ -40,14 +40,32 @@ class SparseTopkParams(ct.Structure):
     ]
 
 
+class _Call:
+    """Checked sizes of a call: its operands, launcher parameters and workspace bytes (none changes afterwards)."""
+
+    __slots__ = ("operands", "params", "nbytes", "launch")
+
+
 @functools.lru_cache(maxsize=64)
-def _launch_state(lib, B, T, TOPK, RATIO, C):
-    """Launcher parameters and workspace bytes of one set of sizes (neither changes afterwards)."""
+def _call(lib, T, C, B, TOPK, RATIO):
+    require(T > 0 and C > 0, "scores must be non-empty")
+    require(C < 2**31, "scores may hold at most 2^31 - 1 columns")
+    require(TOPK > 0, "TOPK must be positive")
+    require(RATIO in (1, 2), "RATIO must be 1 or 2")
+    require(B > 0, "cu_seqlens_q must hold B + 1 offsets")
+    call = _Call()
+    i32 = torch.int32
+    call.operands = (Operand("scores", (T, C), torch.float32), Operand("cu_seqlens_q", (B + 1,), i32),
+                     Operand("seqused_cmp_kv", (B,), i32), Operand("cmp_residual_kv", (B,), i32),
+                     Operand("cmp_sparse_indices", (T, 1, TOPK), i32))
     params = SparseTopkParams(B, T, TOPK, RATIO, C)
     nbytes = ct.c_uint64(0)
     _native.check(lib.workspace_size_sparse_topk_indices_split(ct.byref(nbytes), ct.byref(params)),
                   "workspace_size_sparse_topk_indices_split")
-    return ct.pointer(params), nbytes.value
+    call.params = ct.pointer(params)
+    call.nbytes = nbytes.value
+    call.launch = lib.launch_sparse_topk_indices_split
+    return call
 
 
 def sparse_topk_indices(scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, TOPK=512, RATIO=2, out=None):
@@ -59,45 +77,19 @@ def sparse_topk_indices(scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, T
     """
     require(isinstance(scores, torch.Tensor) and scores.dim() == 2, "scores must be a [T, C] tensor")
     t, c = scores.shape
-    require(t > 0 and c > 0, "scores must be non-empty")
-    require(c < 2**31, "scores may hold at most 2^31 - 1 columns")
-    require(TOPK > 0, "TOPK must be positive")
-    require(RATIO in (1, 2), "RATIO must be 1 or 2")
-    device = scores.device
-    check_tensor("scores", scores, (t, c), torch.float32)
-    b = cu_seqlens_q.numel() - 1
-    require(b > 0, "cu_seqlens_q must hold B + 1 offsets")
-    check_tensor("cu_seqlens_q", cu_seqlens_q, (b + 1,), torch.int32, device)
-    check_tensor("seqused_cmp_kv", seqused_cmp_kv, (b,), torch.int32, device)
-    check_tensor("cmp_residual_kv", cmp_residual_kv, (b,), torch.int32, device)
+    call = _call(_native.library(), t, c, cu_seqlens_q.numel() - 1, TOPK, RATIO)
     if out is None:
-        out = torch.empty((t, 1, TOPK), dtype=torch.int32, device=device)
-    check_tensor("cmp_sparse_indices", out, (t, 1, TOPK), torch.int32, device)
-    check_disjoint(
-        [
-            ("scores", scores, False),
-            ("cu_seqlens_q", cu_seqlens_q, False),
-            ("seqused_cmp_kv", seqused_cmp_kv, False),
-            ("cmp_residual_kv", cmp_residual_kv, False),
-            ("cmp_sparse_indices", out, True),
-        ]
-    )
-    lib = _native.library()
-    params, nbytes = _launch_state(lib, b, t, TOPK, RATIO, c)
-    # Entries of split rows; the caching allocator keeps the block for this stream.
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
-    status = lib.launch_sparse_topk_indices_split(
-        stream_handle(device),
-        scores.data_ptr(),
-        cu_seqlens_q.data_ptr(),
-        seqused_cmp_kv.data_ptr(),
-        cmp_residual_kv.data_ptr(),
-        out.data_ptr(),
-        None if workspace is None else workspace.data_ptr(),
-        nbytes,
-        params,
-    )
-    _native.check(status, "launch_sparse_topk_indices_split")
+        out = torch.empty((t, 1, TOPK), dtype=torch.int32, device=scores.device)
+    device, (s, cu, seq, residual, indices) = operand_pointers(
+        call.operands, (scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, out), 4)
+    workspace = None
+    if call.nbytes:
+        # Entries of split rows; the caching allocator keeps the block for this stream.
+        scratch = torch.empty(call.nbytes, dtype=torch.uint8, device=scores.device)
+        workspace = scratch.data_ptr()
+    status = call.launch(raw_stream(device), s, cu, seq, residual, indices, workspace, call.nbytes, call.params)
+    if status:
+        _native.check(status, "launch_sparse_topk_indices_split")
     return out
 
 
