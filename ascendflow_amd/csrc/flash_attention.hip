@@ -40,8 +40,13 @@ struct FaArgs {
 // Flash-attention forward for D = 128. One workgroup of NW waves owns BQ =
 // NW * QT * 16 query rows of one (batch, head); each wave owns QT 16-row query
 // tiles with Q resident in registers. K and V stream in KC-key chunks through
-// a 3-stage LDS ring filled by the load-to-LDS path two chunks ahead (rows
-// XOR-swizzled on the global side, unit u of row r at u ^ (r & 15)).
+// an LDS ring filled by the load-to-LDS path (rows XOR-swizzled on the global
+// side, unit u of row r at u ^ (r & 15)): three slots each for NW = 8, K and V
+// two chunks ahead; two for NW = 4, K two chunks ahead and V one, so that two
+// workgroups fit a CU (128- or 64-row tiles: less of a ragged, short or causal
+// problem is padding, and one workgroup's start and barriers run under the
+// other's work; per row of a long one K and V are loaded two or four times as
+// often, and 8192 x 8192 takes 990 / 1062 / 1350 us at 256 / 128 / 64 rows).
 // S^T[keys, queries] = K * Q^T and O^T[d, queries] += V^T * P^T run on
 // v_mfma_f32_16x16x32_{f16,bf16}; V^T fragments come through
 // ds_read_b64_tr_b16. Per chunk c the QK MFMAs of chunk c + 1 are issued
@@ -61,7 +66,6 @@ struct FaArgs {
 // visible to query i iff j <= i (top-left); they are applied only in chunks
 // that reach the tail or the diagonal.
 template <int DT> __device__ constexpr float fa_tau() { return DT == DT_F16 ? 8.0f : 0.0f; }
-constexpr int FA_NSTAGE = 3;
 // Progress-ordered wave priorities: a wave starts each chunk at priority 3
 // and steps down at half of QK, after QK and at half of PV, so of the two waves
 // sharing a SIMD the one behind wins the MFMA arbitration (otherwise the older
@@ -70,7 +74,7 @@ constexpr int FA_NSTAGE = 3;
 constexpr bool FA_PROGRESS_PRIO = true;
 
 template <int DT, int NW, int QT>
-__global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_forward_kernel(FaArgs a) {
   typedef typename B16<DT>::scalar scalar;
   typedef typename B16<DT>::x8 x8;
   typedef typename B16<DT>::x4 x4;
@@ -79,21 +83,33 @@ __global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
   constexpr int KT = KC / 16;                  // key tiles per chunk
   constexpr int TILE = KC * ROW_BYTES;         // bytes of one K or V tile
   constexpr int BQ = NW * QT * 16;
+  constexpr int NS = NW == 8 ? 3 : 2;          // ring slots per tensor
   constexpr int ROWS_PER_LOAD = 64 / UNITS;    // rows one wave load covers
   constexpr int LOADS = KC / ROWS_PER_LOAD / NW;  // wave loads per tensor per chunk
   static_assert(LOADS * ROWS_PER_LOAD * NW == KC, "a chunk must split evenly over the waves");
 
-  __shared__ __attribute__((aligned(16))) uint8_t kv_lds[FA_NSTAGE][2][TILE];  // [stage][K, V]
+  __shared__ __attribute__((aligned(16))) uint8_t kv_lds[NS][2][TILE];  // [slot][K, V]
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int g = lane >> 4, i16 = lane & 15;
   const int64_t q_tiles = (a.Sq + BQ - 1) / BQ;
-  const uint32_t logical = xcd_contiguous(blockIdx.x, gridDim.x);
-  // Causal: the longest tiles (largest query rows) get the lowest ids.
-  int64_t qtile = (int64_t)(logical % q_tiles);
-  if (a.causal) qtile = q_tiles - 1 - qtile;
-  const int64_t bh = logical / q_tiles;
+  int64_t qtile, bh;
+  if (a.causal) {
+    // Tiles of all heads from the longest down. The dispatcher deals workgroups
+    // to an XCD's shader engines in turn, so with a head's tiles in a row and
+    // an even number of them, engine 0 got the long ones of every head (B2
+    // HQ32 S1987 126 -> 84 us; B1 HQ32 S4096 211 -> 147; S8192 564 -> 549). Heads that share a
+    // KV head stay on one XCD (blocks go to XCD blockIdx % 8).
+    const uint32_t heads = (uint32_t)a.B * (uint32_t)a.HQ;
+    const uint32_t level = blockIdx.x / heads, i = blockIdx.x % heads;
+    qtile = q_tiles - 1 - level;
+    bh = (heads & 7u) ? i : (i & 7u) * (heads >> 3) + (i >> 3);
+  } else {
+    const uint32_t logical = xcd_contiguous(blockIdx.x, gridDim.x);
+    qtile = (int64_t)(logical % q_tiles);
+    bh = logical / q_tiles;
+  }
   const int head = (int)(bh % a.HQ), batch = (int)(bh / a.HQ);
   const int kv_head = head / (a.HQ / a.HKV);
   const int64_t q0 = qtile * BQ;
@@ -124,36 +140,58 @@ __global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
   // ---- KV movement ---------------------------------------------------------
   const uint32_t kv_base = lds_address(kv_lds[0][0]);
   auto tile_address = [&](int chunk, int tensor) {
-    return opaque_uniform(kv_base + (uint32_t)((chunk % FA_NSTAGE) * 2 + tensor) * TILE);
+    return opaque_uniform(kv_base + (uint32_t)((chunk % NS) * 2 + tensor) * TILE);
   };
   // Wave load p of a chunk covers rows [(wave*LOADS + p)*ROWS_PER_LOAD, +ROWS_PER_LOAD);
   // this lane lands on unit (lane % UNITS) of row lane / UNITS and loads unit
-  // (lane % UNITS) ^ (row & 15) of that row.
-  uint32_t load_offset[LOADS];
+  // (lane % UNITS) ^ (row & 15) of that row. Two loads per wave (NW = 8) keep
+  // their offsets in registers; of four, whose registers would spill, loads 1-3
+  // are load 0 with the swizzle's bits 4p flipped, 4p rows on (a wave's rows
+  // then start at a multiple of 16, so the row bits add without carry).
+  constexpr int OFFSETS = LOADS == 2 ? 2 : 1;
+  static_assert(ROWS_PER_LOAD == 4 && (LOADS == 2 || LOADS == 4), "loads of a wave");
+  uint32_t load_offset[OFFSETS];
 #pragma unroll
-  for (int p = 0; p < LOADS; ++p) {
+  for (int p = 0; p < OFFSETS; ++p) {
     const int r = (wave * LOADS + p) * ROWS_PER_LOAD + lane / UNITS;
     load_offset[p] = (uint32_t)(r * ROW_BYTES + (((lane % UNITS) ^ (r & 15)) << 4));
   }
-  auto fetch = [&](int chunk) {
+  // Rows past Sk read the last key instead (masked later).
+  auto tail_offset = [&](int64_t key0, int p) {
+    const int r = (wave * LOADS + p) * ROWS_PER_LOAD + lane / UNITS;
+    const int rr = (int)min((int64_t)r, a.Sk - 1 - key0);
+    return (uint32_t)(rr * ROW_BYTES + (((lane % UNITS) ^ (r & 15)) << 4));
+  };
+  auto fetch = [&](int chunk) {  // K and V (three slots)
     const int64_t key0 = (int64_t)chunk * KC;
     const char* kbase = K + key0 * ROW_BYTES;
     const char* vbase = V + key0 * ROW_BYTES;
     const bool tail = key0 + KC > a.Sk;
 #pragma unroll
     for (int p = 0; p < LOADS; ++p) {
-      uint32_t off = load_offset[p];
-      if (tail) {  // rows past Sk read the last key instead (masked later)
-        const int r = (wave * LOADS + p) * ROWS_PER_LOAD + lane / UNITS;
-        const int rr = (int)min((int64_t)r, a.Sk - 1 - key0);
-        off = (uint32_t)(rr * ROW_BYTES + (((lane % UNITS) ^ (r & 15)) << 4));
-      }
+      uint32_t off = load_offset[p < OFFSETS ? p : 0];
+      if (tail) off = tail_offset(key0, p);
       const uint32_t row0 = (uint32_t)((wave * LOADS + p) * ROWS_PER_LOAD * ROW_BYTES);
       const uint32_t kd = tile_address(chunk, 0) + row0, vd = tile_address(chunk, 1) + row0;
       __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                        :: "s"(kd), "v"(off), "s"(kbase) : "memory");
       __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                        :: "s"(vd), "v"(off), "s"(vbase) : "memory");
+    }
+  };
+  auto fetch_one = [&](int chunk, int tensor) {  // two slots
+    const int64_t key0 = (int64_t)chunk * KC;
+    const char* base = (tensor ? V : K) + key0 * ROW_BYTES;
+    const uint32_t tile = tile_address(chunk, tensor);
+    const bool tail = key0 + KC > a.Sk;
+#pragma unroll
+    for (int p = 0; p < LOADS; ++p) {
+      uint32_t off =
+          p < OFFSETS ? load_offset[p] : (load_offset[0] ^ (uint32_t)(p << 6)) + (uint32_t)(p * 4 * ROW_BYTES);
+      if (tail) off = tail_offset(key0, p);
+      __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                       :: "s"(tile + (uint32_t)((wave * LOADS + p) * ROWS_PER_LOAD * ROW_BYTES)), "v"(off), "s"(base)
+                       : "memory");
     }
   };
 
@@ -270,22 +308,37 @@ __global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
   constexpr int PV_EXP_STEPS = PV_FRAGS / 2 - 1;  // PV steps with exponentials
   static_assert(QK_FRAGS > QK_EXP0, "no QK step left for exponentials");
   f32x4 s_a[KT][QT], s_b[KT][QT];
-  if (chunks > 0) fetch(0);
-  if (chunks > 1) fetch(1);
+  // Three slots: K and V of chunk c+2 go out together. Two: K(c+2), in K(c)'s
+  // place once QK(c) is over, and V(c+1), in V(c-1)'s; V runs one chunk later,
+  // and two workgroups fit a CU.
   if (chunks > 0) {
+    if constexpr (NS == 3) {
+      fetch(0);
+      if (chunks > 1) fetch(1);
+    } else {
+      fetch_one(0, 0);
+      fetch_one(0, 1);
+      if (chunks > 1) fetch_one(1, 0);
+    }
     if (chunks > 1)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * LOADS));  // KV(0) landed, KV(1) may be in flight
+      wait_vmcnt<NS == 3 ? 2 * LOADS : LOADS>();  // chunk 0 landed, the rest may be in flight
     else
-      __builtin_amdgcn_s_waitcnt(0x0F70);
+      wait_vmcnt<0>();
     block_barrier();
     qk_chunk(0, s_a, [](int) {});
   }
   auto iteration = [&](int c, f32x4 (&cur)[KT][QT], f32x4 (&nxt)[KT][QT]) {
-    // KV(c+1) landed (its loads are the only ones in flight); after the
-    // barrier every wave is past PV(c-1), so tile (c+2) % 3 is free.
+    // K(c+1) and V(c) landed (their loads, with V(c+1)'s, are the only ones in
+    // flight); after the barrier every wave is past QK(c) and PV(c-1), whose
+    // slots are free.
     __builtin_amdgcn_s_waitcnt(0x0F70);
     block_barrier();
-    if (c + 2 < chunks) fetch(c + 2);
+    if constexpr (NS == 3) {
+      if (c + 2 < chunks) fetch(c + 2);
+    } else {
+      if (c + 2 < chunks) fetch_one(c + 2, 0);
+      if (c + 1 < chunks) fetch_one(c + 1, 1);
+    }
     if (c >= clean_chunks) mask(c, cur);
 
     x8 pf[QT][KC / 32];
@@ -344,7 +397,7 @@ __global__ __launch_bounds__(NW * 64) void fa_forward_kernel(FaArgs a) {
       }
     };
 
-    // The last chunk also runs a QK, over the stale tile (c + 1) % 3 (no load
+    // The last chunk also runs a QK, over the stale tile of its slot (no load
     // is in flight into it), so that the softmax has one code path; those
     // scores are never read.
     if (FA_PROGRESS_PRIO) __builtin_amdgcn_s_setprio(3);
@@ -869,63 +922,81 @@ __global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16
 using namespace afa;
 
 namespace {
-constexpr int FA_NW = 8, FA_QT = 2;
-
 constexpr int FD_MAX_SPLITS = 64;  // fa_merge_kernel keeps two splits per thread of a row
 constexpr int64_t FA_CUS = 256;
 constexpr int64_t FD_STREAM_BYTES = int64_t(128) << 20;
 
-template <int DT>
-int launch_fa(const FaArgs& a, hipStream_t s) {
-  constexpr int BQ = FA_NW * FA_QT * 16;
-  const int64_t tiles = (a.Sq + BQ - 1) / BQ;
-  const int64_t blocks = tiles * a.B * a.HQ;
+template <int DT, int NW, int QT>
+int launch_forward(const FaArgs& a, hipStream_t s) {
+  constexpr int BQ = NW * QT * 16;
+  const int64_t blocks = (a.Sq + BQ - 1) / BQ * a.B * a.HQ;
   if (blocks > 0x7fffffffLL) return AFA_E_SHAPE;
-  hipLaunchKernelGGL((fa_forward_kernel<DT, FA_NW, FA_QT>), dim3((unsigned)blocks), dim3(FA_NW * 64), 0, s, a);
+  hipLaunchKernelGGL((fa_forward_kernel<DT, NW, QT>), dim3((unsigned)blocks), dim3(NW * 64), 0, s, a);
   return (int)hipGetLastError();
 }
 
+// Forms of the forward kernel, by query rows of a workgroup's tile: 256 rows in
+// eight waves, one workgroup per CU; 128 and 64 in four waves, two per CU.
+constexpr int FA_FORMS = 3;
+constexpr int FA_ROWS[FA_FORMS] = {256, 128, 64};
+template <int DT>
+int launch_fa(const FaArgs& a, int form, hipStream_t s) {
+  return form == 0 ? launch_forward<DT, 8, 2>(a, s)
+                   : form == 1 ? launch_forward<DT, 4, 2>(a, s) : launch_forward<DT, 4, 1>(a, s);
+}
+
 // Form of a call: the packed split kernel (qt row tiles of 16 per workgroup,
-// `splits` key ranges) or the forward kernel (qt = 0).
+// `splits` key ranges) or a forward kernel (qt = 0).
 struct FaPlan {
   int qt, splits;
   int64_t row_tiles;
+  int form;  // qt = 0
 };
 
 // Picks the cheaper form by a model of MI355X in microseconds (times measured
-// on grids from 16 to 1500 workgroups, bf16), fixed at 256 CUs so that the
-// workspace size depends on the sizes alone. Both kernels run one workgroup
-// per CU:
-//  - forward kernel: FORWARD_STEP per 64-key chunk of a 256-row tile, and
-//    FORWARD_START per workgroup (Q, first loads, output);
-//  - split kernel: a step of four 32-key tiles costs the larger of
-//    SPLIT_STEP[qt] (the latency of 64 KiB of loads, then the waves' own chain
-//    of MFMAs and softmax) and KV_STEP, its 64 KiB when all CUs load at once
-//    (6.9 TB/s), shared by the row tiles that read the same keys; SPLIT_START
-//    for the first workgroup of a CU, ROUND + ROUND_QT * qt for each later one
-//    (its first loads, and the waves' O through LDS), MERGE + MERGE_SPLIT
-//    per split for the second kernel.
-// A causal grid runs at least its longest tile and at most twice the mean.
-// Measured either side of the line (us, split / forward kernel): B1 HQ8 Sq1024
-// causal 18.4 / 36.6, B1 HQ32 HKV8 Sq1000 causal 56 / 37, B1 HQ32 HKV8 Sq256
-// Sk8192 96 / 224, B1 HQ32 HKV8 Sq2000 193 / 73.
+// on grids from 16 to 4096 workgroups, bf16), fixed at 256 CUs so that the
+// workspace size depends on the sizes alone:
+//  - forward kernel: per 64-key chunk ALONE while a CU runs one workgroup of it
+//    (its longest tile then sets the time) and FULL while it runs all that
+//    fit; FORWARD_START for a workgroup's Q, first loads and output;
+//  - split kernel, one workgroup per CU: a step of four 32-key tiles costs the
+//    larger of SPLIT_STEP[qt] (the latency of 64 KiB of loads, then the waves'
+//    own chain of MFMAs and softmax) and KV_STEP, its 64 KiB when all CUs load
+//    at once (6.9 TB/s), shared by the row tiles that read the same keys;
+//    SPLIT_START for the first workgroup of a CU, ROUND + ROUND_QT * qt for
+//    each later one (its first loads, and the waves' O through LDS), MERGE +
+//    MERGE_SPLIT per split for the second kernel.
+// A causal grid runs at least its longest tile and about half of a full one's
+// work. Measured either side of the lines (us; forward kernel of 256 / 128 / 64
+// rows, best split form): B1 HQ8 S1024 causal 37 / 27 / 19.1, 18.3; B1 HQ32 S700
+// causal 27 / 20 / 16, 36; B1 HQ32 HKV8 Sq256 Sk8192 228 / 173 / 125, 93; B3 HQ28
+// S1500 causal 77 / 68 / 82; B2 HQ32 S2048 139 / 146 / 179; B2 HQ32 S5401 causal
+// 564 / 523 / 660; B6 HQ32 S429 42 / 35 / 37, 100; B2 HQ28 S158 11.6 / 9.9 / 6.9, 15.
 // with_splits: there is a workspace for partial results.
 FaPlan choose_fa(const FaArgs& a, bool with_splits) {
-  constexpr double FORWARD_STEP = 1.65, FORWARD_START = 8.0;
-  constexpr double KV_STEP = 2.4, SPLIT_START = 10.0, ROUND = 3.0, ROUND_QT = 1.6, MERGE = 3.0, MERGE_SPLIT = 0.12;
+  constexpr int PER_CU[FA_FORMS] = {1, 2, 2};
+  constexpr double ALONE[FA_FORMS] = {1.7, 1.25, 0.95}, FULL[FA_FORMS] = {1.8, 1.85, 1.3};
+  constexpr double FORWARD_START[FA_FORMS] = {8.0, 6.5, 5.5};
+  constexpr double KV_STEP = 2.4, SPLIT_START = 8.0, ROUND = 3.0, ROUND_QT = 1.6, MERGE = 3.0, MERGE_SPLIT = 0.12;
   constexpr double SPLIT_STEP[FD_MAX_QT + 1] = {0, 1.4, 1.55, 2.0, 2.45};
   const int64_t group = a.HQ / a.HKV, kv_heads = (int64_t)a.B * a.HKV, rows = group * a.Sq;
   const int64_t keys = a.causal ? std::min(a.Sk, a.Sq) : a.Sk;
-  // Time of `blocks` workgroups whose longest takes `steps` steps.
-  auto grid_cost = [&](int64_t blocks, int64_t row_tiles_per_head, double steps, double step, double round) {
-    const double rounds = std::ceil((double)blocks / FA_CUS);
-    const double mean = a.causal && row_tiles_per_head > 1 ? 0.5 * (1 + 1.0 / row_tiles_per_head) : 1.0;
-    return (rounds - 1) * round + std::max(1.0, rounds * mean) * steps * step;
-  };
-  const int64_t forward_tiles = (a.Sq + 255) / 256;
-  FaPlan plan{0, 1, 0};
-  double best = FORWARD_START + grid_cost(forward_tiles * a.B * a.HQ, forward_tiles, std::ceil(keys / 64.0),
-                                          FORWARD_STEP, FORWARD_START);
+  // Mean tile length over the longest, with n row tiles per head.
+  auto mean = [&](int64_t n) { return a.causal && n > 1 ? 0.5 * (1 + 1.0 / n) : 1.0; };
+  FaPlan plan{0, 1, 0, 0};
+  double best = 0;
+  for (int form = 0; form < FA_FORMS; ++form) {
+    const int64_t tiles = (a.Sq + FA_ROWS[form] - 1) / FA_ROWS[form], blocks = tiles * a.B * a.HQ;
+    const double chunks = std::ceil(keys / 64.0), slots = (double)FA_CUS * PER_CU[form];
+    const double cost = FORWARD_START[form] * (0.5 + 0.5 * std::ceil(blocks / slots)) +
+                        std::max(chunks * ALONE[form],
+                                 (a.causal ? blocks / slots : std::ceil(blocks / slots)) * mean(tiles) * chunks * FULL[form] *
+                                     std::min(1.0, std::max(blocks / slots, 1.0 / PER_CU[form])));
+    if (form == 0 || cost < best) {
+      best = cost;
+      plan.form = form;
+    }
+  }
   for (int qt = 1; qt <= FD_MAX_QT; ++qt) {
     const int64_t row_tiles = (rows + 16 * qt - 1) / (16 * qt);
     if (qt > 1 && rows <= 16 * (qt - 1)) break;  // no fewer tiles than with qt - 1
@@ -937,14 +1008,15 @@ FaPlan choose_fa(const FaArgs& a, bool with_splits) {
     const int64_t most = with_splits ? std::min<int64_t>(FD_MAX_SPLITS, std::max<int64_t>(1, key_tiles / FD_WAVES)) : 1;
     for (int64_t splits = 1; splits <= most; ++splits) {
       const int64_t blocks = items * splits;
-      const double active = std::min<double>(1.0, (double)blocks / FA_CUS);
+      const double rounds = std::ceil((double)blocks / FA_CUS), active = std::min<double>(1.0, (double)blocks / FA_CUS);
       const double steps = std::ceil((double)key_tiles / splits / FD_WAVES);
       const double cost = SPLIT_START + (splits > 1 ? MERGE + MERGE_SPLIT * splits : 0.0) +
-                          grid_cost(blocks, (a.Sq + 16 * qt - 1) / (16 * qt), steps,
-                                    std::max(SPLIT_STEP[qt], KV_STEP * active / row_tiles), ROUND + ROUND_QT * qt);
+                          (rounds - 1) * (ROUND + ROUND_QT * qt) +
+                          std::max(1.0, rounds * mean((a.Sq + 16 * qt - 1) / (16 * qt))) * steps *
+                              std::max(SPLIT_STEP[qt], KV_STEP * active / row_tiles);
       if (cost < best) {
         best = cost;
-        plan = FaPlan{qt, (int)splits, row_tiles};
+        plan = FaPlan{qt, (int)splits, row_tiles, 0};
       }
     }
   }
@@ -1014,7 +1086,7 @@ FaArgs make_fa(const void* Q, const void* K, const void* V, void* O, int64_t Sq,
 }
 
 int dispatch_fa(const FaArgs& a, const FaPlan& plan, void* workspace, int dtype, hipStream_t s) {
-  if (plan.qt == 0) return dtype == AFA_DTYPE_F16 ? launch_fa<DT_F16>(a, s) : launch_fa<DT_BF16>(a, s);
+  if (plan.qt == 0) return dtype == AFA_DTYPE_F16 ? launch_fa<DT_F16>(a, plan.form, s) : launch_fa<DT_BF16>(a, plan.form, s);
   return dtype == AFA_DTYPE_F16 ? launch_split<DT_F16>(a, plan, workspace, s)
                                 : launch_split<DT_BF16>(a, plan, workspace, s);
 }

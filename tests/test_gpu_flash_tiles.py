@@ -1,0 +1,41 @@
+"""The forward flash-attention kernel in tiles of 128 and 64 query rows (four
+waves, two slots per tensor in the KV ring): one, two and more key chunks, a
+ragged last one, tiles either side of their rows, causal and grouped heads,
+against the online oracle at the contract tolerance of test_gpu_flash.py."""
+
+import numpy as np
+import pytest
+
+from oracle.attention import inputs
+from tests.test_gpu_flash import assert_contract, online_rows, run_fa
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+    "b,hq,hkv,sq,sk,dtype,causal,case",
+    [
+        # 64-row tiles (small grids)
+        (1, 8, 8, 64, 1, "f16", False, "standard"),
+        (2, 8, 2, 65, 64, "bf16", False, "standard"),
+        (2, 8, 2, 129, 65, "f16", False, "sharp"),
+        (1, 2, 2, 63, 191, "bf16", True, "standard"),
+        (1, 4, 1, 700, 300, "bf16", True, "sharp"),
+        (2, 8, 2, 300, 300, "f16", True, "standard"),
+        # 128-row tiles (more heads than two rounds of 64-row tiles)
+        (48, 8, 8, 257, 64, "bf16", True, "standard"),
+        (40, 16, 16, 129, 65, "f16", False, "standard"),
+        (40, 16, 4, 127, 128, "bf16", False, "sharp"),
+        (48, 8, 8, 120, 193, "f16", False, "standard"),
+        (64, 8, 8, 129, 129, "bf16", True, "standard"),
+    ],
+)
+def test_tiles_match_the_reference_contract(device, b, hq, hkv, sq, sk, dtype, causal, case):
+    print(f"\n[fa tiles] b={b} hq={hq} hkv={hkv} sq={sq} sk={sk} {dtype} causal={causal} case={case}", flush=True)
+    data = inputs(b, hq, hkv, sq, sk, dtype, scale=0.5, case=case)
+    actual = run_fa(data, dtype, causal, device)
+    rows = np.array(sorted({min(r, sq - 1) for r in (0, 15, 16, 62, 63, 64, 127, 128, sq // 2, sq - 1)}))
+    few = [0, b // 2, b - 1] if b > 3 else list(range(b))  # every batch entry is finite, these are compared
+    assert np.isfinite(actual).all()
+    expected = online_rows(data["q"][few], data["k"][few], data["v"][few], rows, dtype, causal, 64)
+    assert_contract(actual[few][:, :, rows], expected, dtype)
