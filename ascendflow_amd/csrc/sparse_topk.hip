@@ -14,24 +14,27 @@
 // The selection works on a monotonic 32-bit key of each score. Three kernels:
 // sparse_topk_row keeps a row in registers (calls of few tokens, rows up to 32K
 // positions; longer ones split into segments and merged), described at its
-// definition; the other two stream a row per workgroup. sparse_topk_filter (rows up to 256K positions; 256 threads up
-// to 32K positions, 1024 beyond):
+// definition; the other two stream a row per workgroup. sparse_topk_filter (rows up
+// to 256K positions; 256 threads up to 32K positions, 1024 beyond):
 //   1. sample: four keys per thread (two in the 1024-thread form: 2048
 //      keys), in blocks of 16 consecutive positions
 //      evenly spaced over the row (issued with the request lookup, over the
 //      whole allocated row, and kept when the token's candidates cover at
 //      least half of it; shorter rows are sampled again over their
-//      candidates); a two-digit radix selection on the sample (the top 22
-//      bits of the key: an estimate needs no more) gives an estimate of the
-//      threshold, taken at 1.25x the expected rank plus 8 (256 threads) or
+//      candidates); one histogram of the sample, linear in the score over its
+//      range, or a two-digit radix selection (the 1024-thread form, and
+//      samples with no usable range), gives an estimate of the threshold, taken at 1.25x the expected rank plus 8 (256 threads) or
 //      twice it plus 16 (1024), so that somewhat more than `take` keys reach
 //      it;
 //   2. filter: one streaming pass over the row (16-byte loads, several in
 //      flight per thread) appends every key >= estimate, with its position,
 //      to an LDS buffer (wave ballots, one LDS atomic per wave and step);
-//   3. exact selection: radix selection (digits of 11, 11 and 10 bits, LDS
-//      histograms) over the buffer, giving the threshold key and how many keys
-//      equal to it are taken; if fewer than `take` keys reached the estimate,
+//   3. exact selection over the buffer: one linear histogram and a ranking of
+//      the few keys in the bin of the take-th, or a radix selection (digits of
+//      11, 11 and 10 bits; the 1024-thread form, and fuller bins), giving the
+//      threshold key and how many keys equal to it are taken (linear instead
+//      of radix: 4096 rows of 16391 83.5 -> 78.6 us, 8192 of 16K 133.9 ->
+//      127.4, 4096 of 4K 35.2 -> 32.7); if fewer than `take` keys reached the estimate,
 //      or the buffer overflowed, the row is filtered again at another sample
 //      rank (binary search, up to four passes), and failing that the same
 //      selection runs over the whole row, re-reading it per digit (same
@@ -299,65 +302,53 @@ __device__ __forceinline__ uint32_t radix_select(ForEachKey for_each_key, int ra
 // buffer resource of range cand * 4 bytes (loads past it return zeros without
 // touching memory): f(key, position) is called by every thread of the wave
 // together, TK_UNROLL * 4 times per step, with key 0 for a position past the
-// candidates (no score maps to key 0). VEC: 16-byte loads of 4 consecutive
-// positions (rows 16-byte aligned); otherwise 4-byte loads.
-template <int THREADS, bool VEC>
+// candidates (no score maps to key 0). 16-byte loads of 4 consecutive
+// positions: a buffer load of any width needs dword alignment, which every f32
+// row has, whatever C; against 4-byte loads 4096 rows of 16391 take 76.9 us
+// instead of 78.6.
+template <int THREADS>
 __device__ __forceinline__ int stream_position(int base, int j) {
   const int tid = threadIdx.x;
-  return VEC ? base + ((j >> 2) * THREADS + tid) * 4 + (j & 3) : base + j * THREADS + tid;
+  return base + ((j >> 2) * THREADS + tid) * 4 + (j & 3);
 }
 
 // The same pass handing each step's UNROLL * 4 keys to f at once:
 // f(keys, base), keys[j] being the key of position stream_position(base, j).
-template <int THREADS, bool VEC, int UNROLL, typename F>
+template <int THREADS, int UNROLL, typename F>
 __device__ __forceinline__ void stream_row_steps(__amdgpu_buffer_rsrc_t rsrc, int cand, F f) {
   constexpr int STEP = THREADS * 4 * UNROLL;
   for (int base = 0; base < cand; base += STEP) {
     uint32_t w[UNROLL * 4];
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u) {
-      if constexpr (VEC) {
-        const u32x4 x = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, stream_position<THREADS, VEC>(base, 4 * u) * 4, 0, 0));
+      const u32x4 x = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, stream_position<THREADS>(base, 4 * u) * 4, 0, 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[4 * u + e] = x[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[4 * u + e] =
-              __builtin_amdgcn_raw_buffer_load_b32(rsrc, stream_position<THREADS, VEC>(base, 4 * u + e) * 4, 0, 0);
-      }
+      for (int e = 0; e < 4; ++e) w[4 * u + e] = x[e];
     }
     uint32_t keys[UNROLL * 4];
 #pragma unroll
     for (int j = 0; j < UNROLL * 4; ++j)
-      keys[j] = stream_position<THREADS, VEC>(base, j) < cand ? score_key(__uint_as_float(w[j])) : 0u;
+      keys[j] = stream_position<THREADS>(base, j) < cand ? score_key(__uint_as_float(w[j])) : 0u;
     f(keys, base);
   }
 }
 
-template <int THREADS, bool VEC, typename F>
+template <int THREADS, typename F>
 __device__ __forceinline__ void stream_row(__amdgpu_buffer_rsrc_t rsrc, int cand, F f) {
   constexpr int STEP = THREADS * 4 * TK_UNROLL;
   for (int base = 0; base < cand; base += STEP) {
     uint32_t w[TK_UNROLL * 4];
 #pragma unroll
     for (int u = 0; u < TK_UNROLL; ++u) {
-      if constexpr (VEC) {
-        const u32x4 x = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, stream_position<THREADS, VEC>(base, 4 * u) * 4, 0, 0));
+      const u32x4 x = __builtin_bit_cast(
+          u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, stream_position<THREADS>(base, 4 * u) * 4, 0, 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[4 * u + e] = x[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[4 * u + e] =
-              __builtin_amdgcn_raw_buffer_load_b32(rsrc, stream_position<THREADS, VEC>(base, 4 * u + e) * 4, 0, 0);
-      }
+      for (int e = 0; e < 4; ++e) w[4 * u + e] = x[e];
     }
 #pragma unroll
     for (int j = 0; j < TK_UNROLL * 4; ++j) {
-      const int p = stream_position<THREADS, VEC>(base, j);
+      const int p = stream_position<THREADS>(base, j);
       f(p < cand ? score_key(__uint_as_float(w[j])) : 0u, p);
     }
   }
@@ -367,6 +358,73 @@ __device__ __forceinline__ int lane_rank(uint64_t mask) {  // set bits of mask b
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
+constexpr uint32_t KEY_LOWEST = 0x00800000u, KEY_HIGHEST = 0xff7fffffu;  // keys of -FLT_MAX and FLT_MAX
+
+__device__ __forceinline__ float key_score(uint32_t k) {  // inverse of score_key, of the nearest finite key
+  k = min(max(k, KEY_LOWEST), KEY_HIGHEST);
+  return __uint_as_float(k ^ ((uint32_t)((int32_t)~k >> 31) | 0x80000000u));
+}
+
+// Maximum over the 64 lanes of a wave (every lane active), in DPP moves as
+// wave_inclusive_scan; lanes shifted in from outside a row keep `v`'s own.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Histogram bins linear in the score over [base, base + span]: non-decreasing
+// in the key; infinities, NaN and keys outside take the end bins.
+struct LinearBins {
+  float base, per_bin;
+  // Over the scores of two keys; false where they span no usable range (none
+  // finite, equal, or too far apart).
+  __device__ __forceinline__ bool set(uint32_t low, uint32_t high) {
+    base = key_score(low);
+    const float span = key_score(high) - base;
+    const bool usable = low <= high && high >= KEY_LOWEST && span > 1e-30f && span < 3e38f;
+    base = usable ? base : 0.f;
+    per_bin = usable ? (TK_BINS - 1) / span : 0.f;  // 0: one bin
+    return usable;
+  }
+  __device__ __forceinline__ void to_scalar() {  // of uniform bins: out of the vector registers
+    base = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(base)));
+    per_bin = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(per_bin)));
+  }
+  __device__ __forceinline__ int of(uint32_t k) const {
+    return (int)fminf(fmaxf((key_score(k) - base) * per_bin, 0.f), (float)(TK_BINS - 1));
+  }
+  // A key that no key of a bin >= b is below (a hundredth of a bin and one
+  // step of the float against the rounding of either direction).
+  __device__ __forceinline__ uint32_t lower_bound(int b) const {
+    if (b <= 0) return 1u;
+    return score_key(base + ((float)b - 0.01f) / per_bin) - 1u;
+  }
+};
+
+// The need-th largest of the `inside` (1..64) keys in LDS, found by every wave of
+// the workgroup for itself; *need becomes how many keys equal to it are taken.
+// Lane l's key is the one when fewer than `need` keys are larger and, with
+// those equal to it, at least `need`.
+__device__ __forceinline__ uint32_t rank_small(const uint32_t* keys, int inside, int lane, int* need) {
+  const uint32_t mine = lane < inside ? keys[lane] : 0u;
+  int larger = 0, equal = 0;
+  for (int i = 0; i < inside; ++i) {
+    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
+    larger += other > mine ? 1 : 0;
+    equal += other == mine ? 1 : 0;
+  }
+  const int owner = (int)__builtin_ctzll(__ballot(lane < inside && larger < *need && larger + equal >= *need));
+  const uint32_t key = (uint32_t)__builtin_amdgcn_readlane((int)mine, owner);
+  *need -= __builtin_amdgcn_readlane(larger, owner);
+  return key;
+}
+constexpr int TK_SMALL = 64;  // keys of a histogram bin that rank_small takes
+
 template <bool COMPACT> struct BufferPosition { typedef int type; };
 template <> struct BufferPosition<true> { typedef uint16_t type; };
 
@@ -374,9 +432,12 @@ template <> struct BufferPosition<true> { typedef uint16_t type; };
 // and buffer positions, so that more workgroups fit in a CU's LDS.
 // Eight waves per SIMD (at most 64 VGPRs): two 1024-thread or eight 256-thread
 // workgroups per CU, as many as the LDS holds.
-template <int THREADS, bool VEC>
+template <int THREADS>
 __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
   constexpr bool COMPACT = THREADS <= 256;
+  // Linear histograms (below); the 1024-thread form, at its register budget,
+  // keeps the radix digits (384 rows of 64K 32.8 us, with them 33.6).
+  constexpr bool LINEAR = COMPACT;
   // 4-position groups per thread and step of the filter pass.
   constexpr int FILTER_UNROLL = THREADS <= 256 ? TK_UNROLL : TK_UNROLL / 2;
   typedef typename BufferPosition<COMPACT>::type Position;
@@ -395,6 +456,11 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
   __shared__ int scan_scratch[2 * THREADS / 64];
   __shared__ int reached;
   __shared__ int request_lds[4];
+  // Uses of LDS that is idle then (292 bytes more and rows of about 24K fit
+  // seven workgroups per CU instead of eight): each wave's range of sample keys
+  // in the buffer, the count of rank_small's keys in the request's place.
+  uint32_t* const range_lds = buf_key;
+  int* const small_count = request_lds;
   constexpr int WAVES = THREADS / 64;
   const int token = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -493,15 +559,55 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
       sample_mask |= i < samples ? 1u << j : 0u;
     }
   }
+  // Range of the sample's finite keys.
+  uint32_t low = 0xffffffffu, high = 0u;
+  if constexpr (LINEAR) {
+#pragma unroll
+    for (int j = 0; j < SPT; ++j)
+      if ((sample_mask >> j) & 1u) {
+        if (sample[j] >= KEY_LOWEST) low = min(low, sample[j]);
+        if (sample[j] <= KEY_HIGHEST) high = max(high, sample[j]);
+      }
+    low = ~wave_max(~low);
+    high = wave_max(high);
+    if (lane == 0) {
+      range_lds[wave] = low;
+      range_lds[WAVES + wave] = high;
+    }
+  }
   for (int i = tid; i < 2 * words; i += THREADS) bitmaps[i] = 0u;
   for (int i = tid; i < RadixLds<COMPACT>::WORDS; i += THREADS) radix.hist[0][i] = 0u;
   if (tid == 0) reached = 0;
   __syncthreads();
+  if (LINEAR && tid == 0) *small_count = 0;  // every thread has read the request
+  LinearBins bins{0.f, 0.f};
+  bool linear = false;  // uniform
+  if constexpr (LINEAR) {
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      low = min(low, range_lds[w]);
+      high = max(high, range_lds[WAVES + w]);
+    }
+    low = (uint32_t)__builtin_amdgcn_readfirstlane((int)low);
+    high = (uint32_t)__builtin_amdgcn_readfirstlane((int)high);
+    linear = bins.set(low, high) && take <= CAP;
+    bins.to_scalar();
+  }
+  if (linear) {
+#pragma unroll
+    for (int j = 0; j < SPT; ++j)
+      if ((sample_mask >> j) & 1u) radix.add(0, bins.of(sample[j]), 1);
+    __syncthreads();
+  }
   if (whole_row_sample) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) samples += scan_scratch[WAVES + w];
   }
-  int parity = 0, unused = 0;
+  auto clear_histogram = [&](int which) {  // by the waves other than wave 0
+    for (int i = 4 * (tid - 64); i < RadixLds<COMPACT>::WORDS; i += 4 * (THREADS - 64))
+      *reinterpret_cast<u32x4*>(&radix.hist[which][i]) = u32x4{0u, 0u, 0u, 0u};
+  };
+  int parity = linear ? 1 : 0, unused = 0;  // hist[parity] is clear (hist[1]: from the first round on)
 
   // 2. Filter: keys >= estimate (>= 1, so never a position past the row),
   // the estimate being the rank-th largest sample. A rank whose estimate lets
@@ -516,24 +622,40 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
                             : min(samples, (int)((2 * (int64_t)take * samples) / cand) + 16);
   int too_few = 0, too_many = samples + 1, n = 0;
   bool buffered = false;
+  uint32_t filter_estimate = 0;
   // A filter pass succeeds only when take <= n <= CAP: with take above the
   // buffer's capacity no pass can, so the row goes straight to the whole-row
   // selection below instead of being streamed by every filter round first.
   for (int round = 0; take <= CAP && round < TK_FILTER_ROUNDS; ++round) {
-    const uint32_t estimate = radix_select<THREADS, COMPACT, 2>(
-        [&](auto f) {
+    // From the linear histogram of the sample, unless its bin holds so many
+    // samples (an outlier's range, or many equal scores) that it says little.
+    uint32_t estimate = 0;
+    if (linear) {
+      if (wave == 0) pick_bin<COMPACT, true>(radix, 0, TK_BINS, rank, lane);
+      else if (round == 0) clear_histogram(1);
+      __syncthreads();
+      linear = radix.choice[2] <= 8 + rank / 4;
+      estimate = (uint32_t)__builtin_amdgcn_readfirstlane((int)bins.lower_bound(radix.choice[0]));
+    }
+    if (!linear) {
+      if (LINEAR && parity == 1) __syncthreads();  // every wave has read the choice
+      estimate = radix_select<THREADS, COMPACT, 2>(
+          [&](auto f) {
 #pragma unroll
-          for (int j = 0; j < SPT; ++j)
-            if ((sample_mask >> j) & 1u) f(sample[j]);
-        },
-        rank, radix, parity, &unused);  // ends with a barrier: every read of `reached` is done
-    if (tid == 0) reached = 0;
-    __syncthreads();
+            for (int j = 0; j < SPT; ++j)
+              if ((sample_mask >> j) & 1u) f(sample[j]);
+          },
+          rank, radix, parity, &unused);  // ends with a barrier: every read of `reached` is done
+    }
+    if (!LINEAR || round > 0) {
+      if (tid == 0) reached = 0;
+      __syncthreads();
+    }
     // Appends: per step, each lane counts its keys that reach the estimate, a
     // wave scan gives each lane its first slot, and ONE LDS atomic per wave
     // reserves the wave's slots (an atomic with a returned value per key
     // position and wave serialises the pass: prefill 217 -> 192 µs).
-    stream_row_steps<THREADS, VEC, FILTER_UNROLL>(
+    stream_row_steps<THREADS, FILTER_UNROLL>(
         rsrc, cand, [&](const uint32_t (&keys)[FILTER_UNROLL * 4], int base) {
           int hits = 0;
 #pragma unroll
@@ -549,7 +671,7 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
             if (keys[j] >= estimate) {
               if (slot < CAP) {
                 buf_key[slot] = keys[j];
-                buf_pos[slot] = (Position)stream_position<THREADS, VEC>(base, j);
+                buf_pos[slot] = (Position)stream_position<THREADS>(base, j);
               }
               ++slot;
             }
@@ -559,6 +681,7 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
     n = reached;
     if (n >= take && n <= CAP) {
       buffered = true;
+      filter_estimate = estimate;
       break;
     }
     if (n < take)
@@ -574,11 +697,42 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
   int need = 0;
   uint32_t threshold = 0;
   if (buffered) {
-    threshold = radix_select<THREADS>(
-        [&](auto f) {
-          for (int i = tid; i < n; i += THREADS) f(buf_key[i]);
-        },
-        take, radix, parity, &need);
+    int bin = -1, inside = TK_SMALL + 1, rest = take;
+    if (linear) {
+      // One histogram, linear between the estimate and the largest sample:
+      // keys above that share the top bin.
+      bins.set(max(filter_estimate, low), high);
+      bins.to_scalar();
+      for (int i = tid; i < n; i += THREADS) radix.add(parity, bins.of(buf_key[i]), 1);
+      __syncthreads();
+      if (wave == 0) pick_bin<COMPACT, true>(radix, parity, TK_BINS, take, lane);
+      else clear_histogram(parity ^ 1);
+      __syncthreads();
+      parity ^= 1;
+      bin = radix.choice[0];
+      inside = radix.choice[2];
+      rest = take - radix.choice[1];
+    }
+    if (LINEAR && inside <= TK_SMALL) {  // uniform
+      uint32_t* const small_key = radix.hist[parity ^ 1];  // the histogram just read
+      for (int i = tid; i < n; i += THREADS) {
+        const uint32_t k = buf_key[i];
+        if (bins.of(k) == bin) small_key[atomicAdd(small_count, 1)] = k;
+      }
+      __syncthreads();
+      threshold = rank_small(small_key, inside, lane, &rest);
+      need = rest;
+    } else {
+      if (LINEAR) __syncthreads();  // every wave has read the choice
+      threshold = radix_select<THREADS>(
+          [&](auto f) {
+            for (int i = tid; i < n; i += THREADS) {
+              const uint32_t k = buf_key[i];
+              if (bin < 0 || bins.of(k) == bin) f(k);
+            }
+          },
+          rest, radix, parity, &need);
+    }
     for (int i = tid; i < n; i += THREADS) {
       const uint32_t k = buf_key[i];
       const int p = buf_pos[i];
@@ -588,12 +742,12 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
   } else {
     threshold = radix_select<THREADS>(
         [&](auto f) {
-          stream_row<THREADS, VEC>(rsrc, cand, [&](uint32_t k, int) {
+          stream_row<THREADS>(rsrc, cand, [&](uint32_t k, int) {
             if (k != 0u) f(k);
           });
         },
         take, radix, parity, &need);
-    stream_row<THREADS, VEC>(rsrc, cand, [&](uint32_t k, int p) {
+    stream_row<THREADS>(rsrc, cand, [&](uint32_t k, int p) {
       if (k > threshold) atomicOr(&above_bits[p >> 5], 1u << (p & 31));
       else if (k == threshold) atomicOr(&equal_bits[p >> 5], 1u << (p & 31));
     });
@@ -667,39 +821,6 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
 // position order, so ties resolve alike), and give the indices.
 enum { TK_ROW = 0, TK_SEGMENT = 1, TK_MERGE = 2 };
 constexpr int TK_ENTRIES = 2048;  // keys that reach the bound, at most
-constexpr uint32_t KEY_LOWEST = 0x00800000u, KEY_HIGHEST = 0xff7fffffu;  // keys of -FLT_MAX and FLT_MAX
-
-__device__ __forceinline__ float key_score(uint32_t k) {  // inverse of score_key, of the nearest finite key
-  k = min(max(k, KEY_LOWEST), KEY_HIGHEST);
-  return __uint_as_float(k ^ ((uint32_t)((int32_t)~k >> 31) | 0x80000000u));
-}
-
-// Maximum over the 64 lanes of a wave (every lane active), in DPP moves as
-// wave_inclusive_scan; lanes shifted in from outside a row keep `v`'s own.
-__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x111, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x112, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x114, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x118, 0xf, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x142, 0xa, 0xf, false));
-  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x143, 0xc, 0xf, false));
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-// Histogram bins linear in the score over [base, base + span]: non-decreasing
-// in the key; infinities, NaN and keys outside take the end bins.
-struct LinearBins {
-  float base, per_bin;
-  __device__ __forceinline__ int of(uint32_t k) const {
-    return (int)fminf(fmaxf((key_score(k) - base) * per_bin, 0.f), (float)(TK_BINS - 1));
-  }
-  // A key that no key of a bin >= b is below (a hundredth of a bin and one
-  // step of the float against the rounding of either direction).
-  __device__ __forceinline__ uint32_t lower_bound(int b) const {
-    if (b <= 0) return 1u;
-    return score_key(base + ((float)b - 0.01f) / per_bin) - 1u;
-  }
-};
 
 template <int THREADS, int ITEMS, int MODE>
 __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384 ? 6 : 4) void sparse_topk_row(TopkArgs a) {
@@ -707,7 +828,6 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   constexpr int CELLS = GROUPS * WAVES;            // (group, wave) cells, in position order
   constexpr int PER_LANE = (CELLS + 63) / 64;
   constexpr int PER_THREAD = TK_ENTRIES / THREADS;  // entries per thread
-  constexpr int SMALL = 64;
   static_assert(ITEMS % 4 == 0 && (PER_LANE == 1 || WAVES % PER_LANE == 0), "cells of a lane stay in one group");
   static_assert(PER_THREAD * THREADS == TK_ENTRIES, "entries split evenly");
   __shared__ RadixLds<false> radix;
@@ -715,7 +835,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   __shared__ __attribute__((aligned(16))) int entry_pos[TK_ENTRIES];
   __shared__ int request_lds[4];
   __shared__ uint32_t range_lds[2][WAVES];
-  __shared__ uint32_t small_key[SMALL];
+  __shared__ uint32_t small_key[TK_SMALL];
   __shared__ int small_count;
   __shared__ uint32_t cells[PER_LANE * 64];
   const int token = a.first_token + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -821,11 +941,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
     high = max(high, range_lds[1][w]);
   }
   LinearBins bins;
-  bins.base = key_score(low);
-  const float span = key_score(high) - bins.base;
-  // No finite maximum: low > high, or high below the finite keys.
-  const bool linear = low <= high && high >= KEY_LOWEST && span > 1e-30f && span < 3e38f;
-  bins.per_bin = (TK_BINS - 1) / span;
+  const bool linear = bins.set(low, high);
   uint32_t bound = 0u;
   int n = TK_ENTRIES + 1;  // keys that reach the bound
   uint32_t before[GROUPS];
@@ -913,9 +1029,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
       k[e] = i < n ? entry_key[i] : 0u;
       p[e] = entry_pos[i];
     }
-    bins.base = key_score(max(bound, low));
-    const float rest = key_score(high) - bins.base;
-    bins.per_bin = rest > 1e-30f ? (TK_BINS - 1) / rest : 0.f;  // 0: one bin
+    bins.set(max(bound, low), high);
 #pragma unroll
     for (int e = 0; e < PER_THREAD; ++e)
       if (k[e] != 0u) atomicAdd(&radix.hist[1][bins.of(k[e])], 1u);
@@ -928,23 +1042,12 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
     const int bin = radix.choice[0], inside = radix.choice[2];
     int need = take - radix.choice[1];
     uint32_t threshold;
-    if (inside <= SMALL) {  // uniform
+    if (inside <= TK_SMALL) {  // uniform
 #pragma unroll
       for (int e = 0; e < PER_THREAD; ++e)
         if (k[e] != 0u && bins.of(k[e]) == bin) small_key[atomicAdd(&small_count, 1)] = k[e];
       block_barrier();
-      // Every wave ranks them: lane l's key is the threshold when fewer than
-      // `need` keys are larger and, with those equal to it, at least `need`.
-      const uint32_t mine = lane < inside ? small_key[lane] : 0u;
-      int larger = 0, equal = 0;
-      for (int i = 0; i < inside; ++i) {
-        const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, i);
-        larger += other > mine ? 1 : 0;
-        equal += other == mine ? 1 : 0;
-      }
-      const int owner = (int)__builtin_ctzll(__ballot(lane < inside && larger < need && larger + equal >= need));
-      threshold = (uint32_t)__builtin_amdgcn_readlane((int)mine, owner);
-      need -= __builtin_amdgcn_readlane(larger, owner);
+      threshold = rank_small(small_key, inside, lane, &need);
     } else {
       int parity = 0;
       threshold = radix_select<THREADS, false>(
@@ -1100,8 +1203,8 @@ static bool row_fits(int64_t C, int64_t topk) {
 
 // Lines of the form, measured either side (us, register form / streaming form,
 // TOPK 512 unless stated): rows of 8K
-// 2000 24.6 / 25.7, 4096 45.2 / 45.0; of 16K 6000 103.6 / 109.9, 8192 135.6 /
-// 134.5; of 16.4K 1000 39.2 / 44.4, 2000 72.0 / 54.1 (a 32K row's registers half
+// 2000 24.6 / 25.7, 4096 45.2 / 42; of 16K 4096 72.5 / 76, 8192 135.6 /
+// 127.4; of 16.4K 1000 39.2 / 44.4, 2000 72.0 / 52 (a 32K row's registers half
 // empty); of 30K 1000 48.8 / 77.0. Split rows of 128K (8 segments): 64 22.5 /
 // 33.3, 600 118 / 107; of 256K 128 (2048 segments) 56.9 / 90; rows of 64K 6 21.7 /
 // 20.1, 384 47.0 / 32.9. 1961 rows of 2.7K with TOPK 1024, which do not fit the
@@ -1110,7 +1213,7 @@ static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
   TopkPlan plan{};
   const int64_t C = p->C, T = p->T;
   const bool fits = row_fits(C, p->TOPK);
-  const int64_t most = C <= 8192 ? 2048 : C <= 16384 ? 6144 : 1024;
+  const int64_t most = C <= 8192 ? 2048 : C <= 16384 ? 5120 : 1024;
   if (C <= 32768 && T <= most && fits) {
     plan.form = TK_FORM_ROW;
     // One 1024-thread workgroup per CU while every token gets a CU of its own,
@@ -1207,7 +1310,6 @@ static int launch_topk(hipStream_t s, const float* scores, const int32_t* cu_seq
       break;
     }
     case TK_FORM_FILTER: {
-      const bool vec = (params->C % 4 == 0) && (reinterpret_cast<uintptr_t>(scores) % 16 == 0);
       a.words = (int32_t)((a.C + 31) / 32);
       // Buffer: rows up to 32K positions (16-bit positions) hold 2 TOPK entries,
       // between 1024 and 8192, so that little of a CU's LDS is spent on it at the
@@ -1219,15 +1321,9 @@ static int launch_topk(hipStream_t s, const float* scores, const int32_t* cu_seq
       // Rows up to 32K positions: 256 threads, more workgroups per CU; longer
       // rows: 1024 threads, more loads in flight per row.
       if (a.C <= 32768) {
-        if (vec)
-          hipLaunchKernelGGL((sparse_topk_filter<256, true>), grid, dim3(256), dynamic_bytes, s, a);
-        else
-          hipLaunchKernelGGL((sparse_topk_filter<256, false>), grid, dim3(256), dynamic_bytes, s, a);
+        hipLaunchKernelGGL(sparse_topk_filter<256>, grid, dim3(256), dynamic_bytes, s, a);
       } else {
-        if (vec)
-          hipLaunchKernelGGL((sparse_topk_filter<1024, true>), grid, dim3(1024), dynamic_bytes, s, a);
-        else
-          hipLaunchKernelGGL((sparse_topk_filter<1024, false>), grid, dim3(1024), dynamic_bytes, s, a);
+        hipLaunchKernelGGL(sparse_topk_filter<1024>, grid, dim3(1024), dynamic_bytes, s, a);
       }
       break;
     }

@@ -2,7 +2,7 @@
 bit-exact against the oracle at the edges of their sizes: rows either side of
 each register size, both workgroup sizes, TOPK either side of the entries the
 kernel holds, segment edges; and calls of many tokens, which the streaming
-form serves. Scores: normal, heavy ties, constant, infinities and NaN, masked
+form serves (its linear histograms and their radix fallback). Scores: normal, heavy ties, constant, infinities and NaN, masked
 with -inf, one outlier that spans the histogram."""
 
 import ctypes as ct
@@ -58,7 +58,7 @@ def check(device, t, c, topk, kind, ratio=1, short=True, seed=0):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["normal", "ties", "constant", "special", "masked", "lowest", "outlier", "tiny"])
-@pytest.mark.parametrize("t,c,topk", [(3, 4096, 512), (3, 8193, 512), (258, 700, 96), (4, 70001, 512)])
+@pytest.mark.parametrize("t,c,topk", [(3, 4096, 512), (3, 8193, 512), (258, 700, 96), (4, 70001, 512), (2049, 1501, 96)])
 def test_score_distributions(device, t, c, topk, kind):
     check(device, t, c, topk, kind, ratio=2)
 
