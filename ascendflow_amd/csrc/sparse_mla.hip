@@ -607,6 +607,12 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
 #pragma unroll
     for (int p = 0; p < FPW; ++p) entry_next[p] = row_list[list_chunk(chunk) * CHUNK + fw * FPW + p];
   };
+  // Shorter rows: the entries of this thread's pieces, also one step ahead (an
+  // LDS round trip off every fetch: with the above 63.0 -> 61.4 us).
+  auto read_pieces = [&](int chunk) {
+#pragma unroll
+    for (int p = 0; p < FPW; ++p) entry_next[p] = row_list[list_chunk(chunk) * CHUNK + (tid + p * NT) / UNITS];
+  };
   auto fetch = [&](int chunk) {
     const uint32_t tile = tile_address(chunk);
     if constexpr (ROW_LOADS) {
@@ -629,7 +635,7 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
       for (int p = 0; p < PIECES; ++p) {
         const int flat = tid + p * NT;
         const int r = flat / UNITS, upos = flat % UNITS;
-        const uint32_t e = row_list[list_chunk(chunk) * CHUNK + r];
+        const uint32_t e = entry_next[p];
         const char* src = ((e & CMP_BIT) ? cmp : ori) + (size_t)(e & ~CMP_BIT) * ROW_BYTES + ((upos ^ (r & 15)) << 4);
         const uint32_t dst = tile + (uint32_t)((wave * 64 + p * NT) * 16);
         if constexpr (STREAM_KV)
@@ -639,6 +645,7 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
           __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                            :: "s"(dst), "v"(src) : "memory");
       }
+      if (chunk + 1 < chunks) read_pieces(chunk + 1);
     }
   };
   // Pipeline step i: wait for KV(i), barrier, fetch KV(i + AHEAD), then the
@@ -646,6 +653,7 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
   // most the younger batch (KV(i + 1), with a 4-tile ring) is in flight.
   if (fetcher && chunks > 0) {
     if constexpr (ROW_LOADS) read_entries(0);
+    else read_pieces(0);
     fetch(0);
     if (AHEAD > 1 && chunks > 1) {
       fetch(1);
@@ -686,8 +694,12 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
     // ---- 4a. score wave: QK, online softmax, P -------------------------------
     // Here the score waves' step (QK and softmax, plus their share of the
     // fetch unless OWN_FETCH) is the longer one: they get the higher wave
-    // priority (the output waves' instead made decode 6% slower).
-    __builtin_amdgcn_s_setprio(2);
+    // priority over the output wave of their SIMD (the output waves' instead
+    // made decode 6% slower). With 2 + 2 waves and D < 512 a SIMD holds one
+    // wave of either role, of several workgroups, and equal priorities are
+    // better (1403 tokens of 32 heads x 256 f16 67.3 -> 63.0 us; at D = 512,
+    // one workgroup per CU, 55.5 -> 56.0).
+    if constexpr (NQ == 4 || D == 512) __builtin_amdgcn_s_setprio(2);
     // The running max (log2 units) starts at the sink and is raised (with l
     // rescaled here and O rescaled by the output waves) only when a head's max
     // exceeds it by more than TAU. This lane holds S^T rows sigma(4g+i) and
