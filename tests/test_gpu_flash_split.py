@@ -60,3 +60,46 @@ def test_split_entry_refuses_a_small_workspace():
     assert lib.launch_attention_target_split(None, p, p, p, p, p, need.value, 0, 16384, ct.byref(params)) == -2
     assert lib.workspace_size_attention_target_split(ct.byref(need), 8192, 8192, ct.byref(params)) == 0
     assert need.value == 0
+
+
+@pytest.mark.gpu
+def test_split_calls_replay_in_a_graph(device):
+    """Split flash attention and split top-k rows, whose workspaces come from
+    the graph's pool, captured once and replayed on new inputs with eager calls
+    between: each replay equals the eager call bit for bit."""
+    from ascendflow_amd.flash_attention import attention_target
+    from ascendflow_amd.sparse_attention import sparse_topk_indices
+
+    gen = torch.Generator(device=device)
+    gen.manual_seed(3)
+    q = torch.empty((2, 8, 1, 128), dtype=torch.bfloat16, device=device)
+    k, v = (torch.empty((2, 2, 9000, 128), dtype=torch.bfloat16, device=device) for _ in range(2))
+    scores = torch.empty((3, 70000), device=device)
+    i32 = dict(dtype=torch.int32, device=device)
+    meta = (torch.tensor([0, 3], **i32), torch.tensor([70000], **i32), torch.tensor([0], **i32))
+    o, indices = torch.empty_like(q), torch.empty((3, 1, 512), **i32)
+
+    def fill():
+        for t in (q, k, v, scores):
+            t.normal_(generator=gen)
+
+    def calls():
+        attention_target(q, k, v, o, 1, 9000, B=2, HQ=8, HKV=2, D=128, DTYPE="bf16", SCALE=128**-0.5)
+        sparse_topk_indices(scores, *meta, TOPK=512, RATIO=2, out=indices)
+
+    fill()
+    calls()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        calls()
+    for _ in range(3):
+        fill()
+        calls()
+        torch.cuda.synchronize()
+        expected = o.clone(), indices.clone()
+        o.fill_(float("nan"))
+        indices.fill_(-7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, expected[0]) and torch.equal(indices, expected[1])
