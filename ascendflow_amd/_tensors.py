@@ -8,6 +8,9 @@ values, as in the reference (docs/operators/sparse-mla.md:83-84).
 
 from __future__ import annotations
 
+import ctypes as ct
+import functools
+
 import torch
 
 DTYPES = {"bf16": torch.bfloat16, "f16": torch.float16}
@@ -95,6 +98,24 @@ def operand_pointers(operands, tensors, written):
         if p < end and start < p + operands[i].nbytes and i != written:
             check_disjoint([(o.name, t, i == written) for i, (o, t) in enumerate(zip(operands, tensors))])
     return device, pointers
+
+
+_PLAIN = frozenset((bool, int, float, str, ct.CDLL))
+
+
+def kept_by_value(build):
+    """``build(*sizes)``, its last 64 results kept where every argument is a
+    plain number or text (or the library), which nobody can change under the
+    key; 1, 1.0 and True are different keys, since a float is refused where a
+    count is due. Other number-likes (NumPy scalars and arrays, tensors), whose
+    value may change or that have no hash, are built for each call."""
+    kept = functools.lru_cache(maxsize=64, typed=True)(build)
+
+    @functools.wraps(build)
+    def plan(*sizes):
+        return kept(*sizes) if _PLAIN.issuperset(map(type, sizes)) else build(*sizes)
+
+    return plan
 
 
 def raw_stream(device_index) -> int:

@@ -13,12 +13,11 @@ asserts (``attention.py:305-318``) and otherwise ignored.
 from __future__ import annotations
 
 import ctypes as ct
-import functools
 
 import torch
 
 from .. import _native
-from .._tensors import DTYPES, Operand, operand_pointers, raw_stream, require, storage_dtype
+from .._tensors import DTYPES, Operand, kept_by_value, operand_pointers, raw_stream, require, storage_dtype
 
 
 def causal_policy(sq, sk):
@@ -37,7 +36,7 @@ class _Call:
     __slots__ = ("Sq", "Sk", "operands", "params", "nbytes", "launch")
 
 
-@functools.lru_cache(maxsize=64)
+@kept_by_value
 def _call(lib, Sq, Sk, B, HQ, HKV, D, BQ, BM, BK, CK, VR, GROUPS, dtype, SCALE, causal):
     require(Sq >= 1 and Sk >= 1, "Sq and Sk must be >= 1")
     require(B > 0 and HQ > 0 and HKV > 0, "positive batch and head counts")

@@ -7,15 +7,13 @@ P normalised before its FP16 cast. Launches ``launch_simple_attention``.
 
 from __future__ import annotations
 
-import functools
-
 import torch
 
 from .. import _native
-from .._tensors import Operand, operand_pointers, raw_stream, require
+from .._tensors import Operand, kept_by_value, operand_pointers, raw_stream, require
 
 
-@functools.lru_cache(maxsize=64)
+@kept_by_value
 def _operands(S, H, GROUPS):
     """Operands of a call of checked sizes."""
     require(S > 0 and S % 64 == 0, "S must be a positive multiple of 64")

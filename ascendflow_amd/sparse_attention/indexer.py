@@ -22,12 +22,11 @@ framework can trace the indexer -> top-k -> ``sparse_flash_mla`` chain.
 from __future__ import annotations
 
 import ctypes as ct
-import functools
 
 import torch
 
 from .. import _native
-from .._tensors import Operand, operand_pointers, raw_stream, require
+from .._tensors import Operand, kept_by_value, operand_pointers, raw_stream, require
 
 
 class SparseTopkParams(ct.Structure):
@@ -46,7 +45,7 @@ class _Call:
     __slots__ = ("operands", "params", "nbytes", "launch")
 
 
-@functools.lru_cache(maxsize=64)
+@kept_by_value
 def _call(lib, T, C, B, TOPK, RATIO):
     require(T > 0 and C > 0, "scores must be non-empty")
     require(C < 2**31, "scores may hold at most 2^31 - 1 columns")
