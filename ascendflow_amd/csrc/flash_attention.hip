@@ -1006,14 +1006,19 @@ FaPlan choose_fa(const FaArgs& a, bool with_splits) {
     if (a.causal && group > 1 && a.Sq > 256 && a.Sq % (16 * qt)) continue;
     const int64_t key_tiles = (keys + FD_KEYS - 1) / FD_KEYS;
     const int64_t most = with_splits ? std::min<int64_t>(FD_MAX_SPLITS, std::max<int64_t>(1, key_tiles / FD_WAVES)) : 1;
+    const double tile_mean = mean((a.Sq + 16 * qt - 1) / (16 * qt));
+    const double least = std::max(1.0, tile_mean * (double)items * (double)key_tiles / (FA_CUS * FD_WAVES));
     for (int64_t splits = 1; splits <= most; ++splits) {
       const int64_t blocks = items * splits;
       const double rounds = std::ceil((double)blocks / FA_CUS), active = std::min<double>(1.0, (double)blocks / FA_CUS);
+      const double starts = SPLIT_START + (splits > 1 ? MERGE + MERGE_SPLIT * splits : 0.0) +
+                            (rounds - 1) * (ROUND + ROUND_QT * qt);
+      const double step = std::max(SPLIT_STEP[qt], KV_STEP * active / row_tiles);
+      // More splits never make the starts or a step cheaper, and the steps of
+      // all rounds together are at least `least`: none of them beats the best.
+      if (starts + least * step >= best) break;
       const double steps = std::ceil((double)key_tiles / splits / FD_WAVES);
-      const double cost = SPLIT_START + (splits > 1 ? MERGE + MERGE_SPLIT * splits : 0.0) +
-                          (rounds - 1) * (ROUND + ROUND_QT * qt) +
-                          std::max(1.0, rounds * mean((a.Sq + 16 * qt - 1) / (16 * qt))) * steps *
-                              std::max(SPLIT_STEP[qt], KV_STEP * active / row_tiles);
+      const double cost = starts + std::max(1.0, rounds * tile_mean) * steps * step;
       if (cost < best) {
         best = cost;
         plan = FaPlan{qt, (int)splits, row_tiles, 0};
