@@ -45,7 +45,6 @@
 // The row is read once from HBM on the common path. sparse_topk_stream
 // serves longer rows: every digit, and the output, re-read the row.
 #include <algorithm>
-#include <cmath>
 
 #include "common.h"
 #include "../../include/ascendflow_amd.h"
@@ -806,24 +805,37 @@ __global__ __launch_bounds__(THREADS, 8) void sparse_topk_filter(TopkArgs a) {
 //      SMALL of them: radix selection);
 //   4. the entries that are taken, compacted in order, are the output.
 // A row with no usable range (its finite maxima all equal, or none finite) or
-// with more entries than LDS holds (many equal scores; TOPK above about half
-// of TK_ENTRIES) takes the radix selection over the whole row, read again.
-// Measured, call (us, against the streaming forms): 64 rows of 16K 29.8 -> 16,
-// 300 31.5 -> 16, 2000 56.7 -> 40.3, 4096 82.6 -> 72.5; 300 rows of 30K 68.4 ->
-// 20; split, 4 rows of 256K 66 -> 22, of 512K 2,500 -> 22. One 16K row in a
+// with more entries than LDS holds (many equal scores) takes the radix selection
+// over the whole row, read again.
+// The scores buffer may be far wider than a token's candidates (short contexts
+// among long ones, a buffer of the largest size). BOUNDED: the request is looked
+// up first, and loads and work end at the candidates; one round trip more, which
+// several workgroups per CU hide and which the registers of a wide row save
+// anyway. Rows up to 16K of a workgroup that has a CU to itself keep both loads
+// in one round trip. Measured with a quarter of the row as candidates, reading
+// the whole row -> its candidates (us, TOPK 512): 500 rows of 30K 23.5 -> 13.1,
+// 1000 of 16K 21.3 -> 15.3, 256 of 30K 14.9 -> 9.2; full rows 27.1 -> 26.3, 24.3
+// -> 25.0, 16.8 -> 16.5.
+// Measured, GPU time (us, against the streaming form of before): 64 rows of 16K
+// 26.8 -> 9.7, 350 36.5 -> 15.2, 1500 46.3 -> 32.5; 256 rows of 30K 71 -> 16.5; split, 1
+// row of 256K 52 -> 17.5, of 420K 1760 -> 17.7. One 16K row in a
 // 1024-thread workgroup takes 8.2 us: row and lookup 3.3, bound 1.3, entries 1.6,
 // threshold 1.6, output 0.4.
 //
 // ROW: scores to indices. SEGMENT: blockIdx.y is a segment of a longer row;
 // its min(TOPK, candidates) largest go to the workspace as keys and positions
-// in ascending position order, then key 0 up to a.seg_keep entries. MERGE: the
-// segments' entries of a token, in order, are the row (their order is the
-// position order, so ties resolve alike), and give the indices.
+// in ascending position order, then key 0 up to a.seg_keep entries. A token with
+// no candidates past the first segment gets its indices from that segment.
+// MERGE: the segments' entries of any other token, in order, are the row (their
+// order is the position order, so ties resolve alike), and give the indices.
 enum { TK_ROW = 0, TK_SEGMENT = 1, TK_MERGE = 2 };
 constexpr int TK_ENTRIES = 2048;  // keys that reach the bound, at most
+constexpr int TK_SEGMENT_ITEMS = 16;
+constexpr int64_t TK_SEGMENT_SIZE = 1024 * TK_SEGMENT_ITEMS;
 
 template <int THREADS, int ITEMS, int MODE>
 __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384 ? 6 : 4) void sparse_topk_row(TopkArgs a) {
+  constexpr bool BOUNDED = MODE == TK_SEGMENT || (MODE == TK_ROW && (THREADS == 512 || ITEMS > 16));
   constexpr int WAVES = THREADS / 64, GROUPS = ITEMS / 4;
   constexpr int CELLS = GROUPS * WAVES;            // (group, wave) cells, in position order
   constexpr int PER_LANE = (CELLS + 63) / 64;
@@ -841,7 +853,8 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   const int token = a.first_token + (int)blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  // ---- the request (thread b holds request b) and the row, in one round trip ----
+  // ---- the request (thread b holds request b) and the row: in one round trip, or
+  // (BOUNDED) the row's candidates alone once the request is known ---------------
   int begin = 0, next = 0, available = 0, residual = 0;
   const bool early = a.B <= THREADS;  // uniform
   if (early && tid < a.B) {
@@ -854,18 +867,22 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   const int held = MODE == TK_MERGE ? a.segments * a.seg_keep : (int)min<int64_t>(a.C - first, THREADS * ITEMS);
   const uint32_t* source = MODE == TK_MERGE ? a.seg_key + (size_t)blockIdx.x * held
                                             : reinterpret_cast<const uint32_t*>(a.scores) + (size_t)token * a.C + first;
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(source), (short)0, held * 4, BUFFER_WORD3);
-  auto load_group = [&](int u) {  // past the row: zeros, with no memory traffic
+  int reach = held;  // positions that are read
+  auto load_group = [&](int u) {  // past the reach: zeros, with no memory traffic
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(source), (short)0, reach * 4, BUFFER_WORD3);
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (u * THREADS + tid) * 16, 0, 0));
   };
   uint32_t key[ITEMS];  // the score words, then their keys (0: not a candidate)
+  auto load_row = [&]() {
 #pragma unroll
-  for (int u = 0; u < GROUPS; ++u) {
-    const u32x4 x = load_group(u);
+    for (int u = 0; u < GROUPS; ++u) {
+      const u32x4 x = load_group(u);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) key[4 * u + j] = x[j];
-  }
+      for (int j = 0; j < 4; ++j) key[4 * u + j] = x[j];
+    }
+  };
+  if constexpr (!BOUNDED) load_row();
   for (int i = 4 * tid; i < 2 * TK_BINS; i += 4 * THREADS)
     *reinterpret_cast<u32x4*>(&radix.hist[0][0] + i) = u32x4{0u, 0u, 0u, 0u};
   if (tid == 0) small_count = 0;
@@ -893,17 +910,33 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
     seg_key = a.seg_key + at;
     seg_pos = a.seg_pos + at;
     cand = (int)max<int64_t>(0, min<int64_t>(tb.cand - first, held));
-    take = min(take, cand);
-    for (int i = take + tid; i < a.seg_keep; i += THREADS) seg_key[i] = 0u;
-    if (take == 0) return;
+    if (tb.cand <= THREADS * ITEMS) {  // the first segment is the row: its indices are the result
+      if (blockIdx.y != 0 || trivial_selection<THREADS>(a, tb, out)) return;
+    } else {
+      take = min(take, cand);
+      for (int i = take + tid; i < a.seg_keep; i += THREADS) seg_key[i] = 0u;
+      if (take == 0) return;
+    }
   } else {
+    if (MODE == TK_MERGE && tb.cand <= TK_SEGMENT_SIZE) return;  // written by its segment
     if (trivial_selection<THREADS>(a, tb, out)) return;
   }
+  if constexpr (BOUNDED) {
+    reach = __builtin_amdgcn_readfirstlane(cand);
+    load_row();
+  }
+  // What `key` holds that can be nonzero: the candidates, or the entries of the segments with any.
+  const int members = MODE == TK_MERGE ? (cand + (int)TK_SEGMENT_SIZE - 1) / (int)TK_SEGMENT_SIZE * a.seg_keep : cand;
+  auto used = [&](int u) { return !BOUNDED || u * THREADS * 4 < reach; };  // group u holds candidates (uniform)
   auto position = [&](int i) { return ((i >> 2) * THREADS + tid) * 4 + (i & 3); };  // of key[i]
   auto emit = [&](int slot, uint32_t k, int p) {
     if constexpr (MODE == TK_SEGMENT) {
-      seg_key[slot] = k;
-      seg_pos[slot] = (int)first + p;
+      if (tb.cand <= THREADS * ITEMS) {
+        out[slot] = p;
+      } else {
+        seg_key[slot] = k;
+        seg_pos[slot] = (int)first + p;
+      }
     } else if constexpr (MODE == TK_MERGE) {
       out[slot] = a.seg_pos[(size_t)blockIdx.x * held + p];
     } else {
@@ -917,16 +950,18 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
 #pragma unroll
   for (int u = 0; u < GROUPS; ++u) {
     uint32_t m = 0u;
+    if (used(u)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = 4 * u + j;
-      if constexpr (MODE != TK_MERGE) key[i] = position(i) < cand ? score_key(__uint_as_float(key[i])) : 0u;
-      key[i] = opaque(key[i]);  // no comparison is kept in scalar registers for the steps below
-      m = max(m, key[i]);
+      for (int j = 0; j < 4; ++j) {
+        const int i = 4 * u + j;
+        if constexpr (MODE != TK_MERGE) key[i] = position(i) < cand ? score_key(__uint_as_float(key[i])) : 0u;
+        key[i] = opaque(key[i]);  // no comparison is kept in scalar registers for the steps below
+        m = max(m, key[i]);
+      }
+      if (m >= KEY_LOWEST) low = min(low, m);
+      if (m <= KEY_HIGHEST) high = max(high, m);
     }
     top[u] = m;
-    if (m >= KEY_LOWEST) low = min(low, m);
-    if (m <= KEY_HIGHEST) high = max(high, m);
   }
   low = ~wave_max(~low);
   high = wave_max(high);
@@ -948,7 +983,11 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   auto scan_cells = [&](auto count) {  // count(u): this thread's (packed) count of group u, at most 4 in each half
 #pragma unroll
     for (int u = 0; u < GROUPS; ++u) {
-      const int c = count(u), incl = wave_inclusive_scan(c);
+      int c = 0, incl = 0;
+      if (used(u)) {
+        c = count(u);
+        incl = wave_inclusive_scan(c);
+      }
       before[u] = (uint32_t)(incl - c);
       if (lane == 63) cells[u * WAVES + wave] = (uint32_t)incl;
     }
@@ -984,9 +1023,27 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
       }
   };
   if (linear) {  // uniform
+    // By group maxima, m `take` members leave 1.66 `take` keys at the bound for m
+    // = 5 and 1.27 for m = 8, and with fewer groups than `take` all of them; where
+    // that could overflow the entries, the histogram takes every key: little more
+    // than `take` reach the bound (500 rows of 30K with 3.7K candidates and TOPK
+    // 1024 16.6 us, by a radix selection over the row, -> 12.1).
+    if (take > TK_ENTRIES / 4 && members > TK_ENTRIES &&
+        members < (take <= TK_ENTRIES / 2 ? 5 : 8) * (int64_t)take) {  // uniform
 #pragma unroll
-    for (int u = 0; u < GROUPS; ++u)
-      if (top[u] != 0u) atomicAdd(&radix.hist[0][bins.of(top[u])], 1u);
+      for (int u = 0; u < GROUPS; ++u) {
+        if (u * THREADS * 4 >= members) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t k = opaque(key[4 * u + j]);
+          if (k != 0u) atomicAdd(&radix.hist[0][bins.of(k)], 1u);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < GROUPS; ++u)
+        if (top[u] != 0u) atomicAdd(&radix.hist[0][bins.of(top[u])], 1u);
+    }
     block_barrier();
     if (wave == 0) pick_bin<false, true>(radix, 0, TK_BINS, take, lane);
     block_barrier();
@@ -1005,6 +1062,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   if (n <= TK_ENTRIES) {  // uniform
 #pragma unroll
     for (int u = 0; u < GROUPS; ++u) {
+      if (!used(u)) continue;
       int slot, unused;
       cell_base(u, slot, unused);
       slot += (int)before[u];
@@ -1095,7 +1153,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   int parity = 0, need = 0;
   const uint32_t threshold = radix_select<THREADS, false>(
       [&](auto f) {
-        for (int u = 0; u < GROUPS; ++u) {
+        for (int u = 0; u < GROUPS && u * THREADS * 4 < members; ++u) {
           const u32x4 x = load_group(u);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
@@ -1116,6 +1174,7 @@ __global__ __launch_bounds__(THREADS, ITEMS <= 16 ? 8 : THREADS * ITEMS <= 16384
   read_cells();
 #pragma unroll
   for (int u = 0; u < GROUPS; ++u) {
+    if (!used(u)) continue;
     int above, equal;
     cell_base(u, above, equal);
     above += (int)(before[u] & 0xffffu);
@@ -1185,35 +1244,36 @@ struct TopkPlan {
   int segments, keep;  // SPLIT: segments of TK_SEGMENT_SIZE positions, entries kept of each
   int64_t tokens;      // SPLIT: tokens per pair of launches
 };
-constexpr int TK_SEGMENT_ITEMS = 16;
-constexpr int64_t TK_SEGMENT_SIZE = 1024 * TK_SEGMENT_ITEMS;
 constexpr int64_t TK_MERGE_MAX = 1024 * 32;  // entries of all segments of a row
 constexpr int64_t TK_SPLIT_WORKGROUPS = 2048;
 constexpr int64_t TK_SPLIT_BYTES = int64_t(64) << 20;  // workspace of a call, at most (one token at least)
 
-// Whether the keys of a row of C that reach sparse_topk_row's bound are
-// expected to fit its entries: with a fraction f = TOPK / (C / 4) of the groups
-// above the threshold, 1 - (1 - f)^(1/4) of the keys are. Rows that do not fit
-// give the same result through a radix selection, later.
-static bool row_fits(int64_t C, int64_t topk) {
-  if (C <= TK_ENTRIES) return true;
-  const double f = 4.0 * (double)topk / (double)C;
-  return f < 1.0 && (double)C * (1.0 - std::sqrt(std::sqrt(1.0 - f))) <= 0.93 * TK_ENTRIES;
-}
-
-// Lines of the form, measured either side (us, register form / streaming form,
-// TOPK 512 unless stated): rows of 8K
-// 2000 24.6 / 25.7, 4096 45.2 / 42; of 16K 4096 72.5 / 76, 8192 135.6 /
-// 127.4; of 16.4K 1000 39.2 / 44.4, 2000 72.0 / 52 (a 32K row's registers half
-// empty); of 30K 1000 48.8 / 77.0. Split rows of 128K (8 segments): 64 22.5 /
-// 33.3, 600 118 / 107; of 256K 128 (2048 segments) 56.9 / 90; rows of 64K 6 21.7 /
-// 20.1, 384 47.0 / 32.9. 1961 rows of 2.7K with TOPK 1024, which do not fit the
-// entries, 31.1 / 29.6.
+// Lines of the form. A buffer's columns say little of its tokens' candidates, and
+// the streaming form's time follows those more closely; the register form is
+// taken up to where it is faster with half of the columns as candidates and at
+// most about a tenth slower with a quarter, at every share for calls of up to 512
+// tokens (decode, in buffers of its largest context). Measured either side (us,
+// register form / streaming form; all, half, a quarter, an eighth of the columns;
+// TOPK 512 unless stated): 500 rows of 30K 26 / 69, 18 / 37, 13 / 16, 11.3 / 13.2; 1000
+// 45 / 74, 31 / 45, 24 / 22, 20 / 17; 1000 of 20K 0.72x, 0.72x, 1.15x, 1.25x, with TOPK 256
+// 0.98x, 0.98x, 1.07x, 1.34x; 2000 of 16K 40 / 54, 30 / 32, 25 / 23, 24 / 23, 3000 0.82x,
+// 1.00x, 1.10x, 1.11x, 5000 0.86x, 1.08x, 1.18x, 1.20x, with TOPK 1024
+// 0.84x, 0.98x, 0.96x, 0.87x; 2000 of 8K 0.79x, 0.92x, 0.90x, 0.79x; of 700 with TOPK
+// 256 0.91x, 1.16x.
+// Split rows, 64 tokens: of 66K 20.2 / 22.0, 17.1 / 16.0, 16.5 / 12.6; of 100K 22.5 / 28.6,
+// 17 / 19, 16 / 14; of 256K 36 / 98, 25 / 54, 19.3 / 21.1, 17.8 / 15.2; 128 tokens: of 128K 34.7
+// / 33.6; of 256K 58 / 99, 37 / 56, 28 / 22. Candidates past one segment and up to about
+// 40K lose 1 to 5 us to the second launch; up to one segment there is nothing to merge
+// (11.5 / 11.8).
 static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
   TopkPlan plan{};
   const int64_t C = p->C, T = p->T;
-  const bool fits = row_fits(C, p->TOPK);
-  const int64_t most = C <= 8192 ? 2048 : C <= 16384 ? 5120 : 1024;
+  const bool fits = p->TOPK <= 1408;  // entries, whatever the candidates (see the bound)
+  const int64_t most = C > 24576   ? 1024
+                       : C > 16384 ? (p->TOPK > 256 ? 1024 : 512)
+                       : C > 8192  ? (p->TOPK > 512 ? 5120 : p->TOPK > 256 ? 3072 : 2048)
+                       : C > 1024  ? 2048
+                                   : 1024;
   if (C <= 32768 && T <= most && fits) {
     plan.form = TK_FORM_ROW;
     // One 1024-thread workgroup per CU while every token gets a CU of its own,
@@ -1226,8 +1286,9 @@ static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
   }
   const int64_t segments = (C + TK_SEGMENT_SIZE - 1) / TK_SEGMENT_SIZE;
   const int64_t keep = (std::min<int64_t>(p->TOPK, TK_SEGMENT_SIZE) + 3) / 4 * 4;
-  if (with_workspace && C > 65536 && segments * keep <= TK_MERGE_MAX &&
-      (C > TK_FILTER_MAX_C || T * segments <= TK_SPLIT_WORKGROUPS)) {
+  const bool few = T <= 64 || (segments >= 12 && T * segments <= TK_SPLIT_WORKGROUPS);
+  if (with_workspace && segments * keep <= TK_MERGE_MAX &&
+      (C > TK_FILTER_MAX_C || (segments >= 6 && few && fits))) {
     plan.form = TK_FORM_SPLIT;
     plan.segments = (int)segments;
     plan.keep = (int)keep;
