@@ -608,7 +608,12 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
     for (int p = 0; p < FPW; ++p) entry_next[p] = row_list[list_chunk(chunk) * CHUNK + fw * FPW + p];
   };
   // Shorter rows: the entries of this thread's pieces, also one step ahead (an
-  // LDS round trip off every fetch: with the above 63.0 -> 61.4 us).
+  // LDS round trip off every fetch) with 2 + 2 waves, two to four pieces each:
+  // 1403 tokens of 32 heads x 256 64.9 -> 62.3 us, 245 22.9 -> 21.7. With 4 + 4 it
+  // hides no more than it costs (64 heads x 256, 32 tokens 14.6 -> 14.9, 2000
+  // 113 -> 113; x 128, one token 10.2 -> 10.3, 640 30.2 -> 30.3) and the entries
+  // are read where they are used.
+  constexpr bool PIECES_AHEAD = !ROW_LOADS && NQ == 2;
   auto read_pieces = [&](int chunk) {
 #pragma unroll
     for (int p = 0; p < FPW; ++p) entry_next[p] = row_list[list_chunk(chunk) * CHUNK + (tid + p * NT) / UNITS];
@@ -635,7 +640,7 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
       for (int p = 0; p < PIECES; ++p) {
         const int flat = tid + p * NT;
         const int r = flat / UNITS, upos = flat % UNITS;
-        const uint32_t e = entry_next[p];
+        const uint32_t e = PIECES_AHEAD ? entry_next[p] : row_list[list_chunk(chunk) * CHUNK + r];
         const char* src = ((e & CMP_BIT) ? cmp : ori) + (size_t)(e & ~CMP_BIT) * ROW_BYTES + ((upos ^ (r & 15)) << 4);
         const uint32_t dst = tile + (uint32_t)((wave * 64 + p * NT) * 16);
         if constexpr (STREAM_KV)
@@ -645,7 +650,8 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
           __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                            :: "s"(dst), "v"(src) : "memory");
       }
-      if (chunk + 1 < chunks) read_pieces(chunk + 1);
+      if constexpr (PIECES_AHEAD)
+        if (chunk + 1 < chunks) read_pieces(chunk + 1);
     }
   };
   // Pipeline step i: wait for KV(i), barrier, fetch KV(i + AHEAD), then the
@@ -653,7 +659,7 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
   // most the younger batch (KV(i + 1), with a 4-tile ring) is in flight.
   if (fetcher && chunks > 0) {
     if constexpr (ROW_LOADS) read_entries(0);
-    else read_pieces(0);
+    else if constexpr (PIECES_AHEAD) read_pieces(0);
     fetch(0);
     if (AHEAD > 1 && chunks > 1) {
       fetch(1);
