@@ -145,10 +145,11 @@ __device__ __forceinline__ uint32_t opaque_uniform(uint32_t v) {
 // expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14, all other fields at max).
 constexpr int WAIT_LGKM0 = 0xC07F;
 // s_waitcnt vmcnt(N) alone: wait until at most N vector memory operations of
-// this wave are in flight. The kernels use N > 0 only where every operation in
-// flight is a load (loads and loads to LDS retire in issue order, so this waits
-// for all but the N most recent); behind stores they wait with N = 0, since
-// stores are not relied on to retire in order with loads.
+// this wave are in flight. Loads and loads to LDS retire in issue order among
+// themselves, so while a load is in flight the loads issued after it are too:
+// with N of those the wait is enough for it, whatever stores are in flight
+// besides (they count as well and can only make it longer). Nothing is assumed
+// about the order of stores against loads: a wait for a store is N = 0.
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt holds 6 bits");

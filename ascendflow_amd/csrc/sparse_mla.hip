@@ -80,7 +80,6 @@ struct SparseArgs {
   int32_t split_from;    // first split (token, head tile) key; keys below it run whole
   int32_t ring;          // KV ring tiles of the persistent kernel (3 or 4)
   int32_t stream_kv;     // few query tokens per request: non-temporal KV, Q and O accesses (D = 512)
-  int32_t write_plan;    // one-item kernel: leave the row lists in plan_count / plan_rows
   float scale;
 };
 
@@ -449,8 +448,11 @@ constexpr int LOOK_QK = 5;  // KV fragment lookahead (k-steps) of a score wave
 // wait at the barrier (decode B64 x 6 ~2% faster than every wave fetching 4
 // rows); other shapes spread the fetch over every wave.
 // STREAM_KV: KV row loads are non-temporal as well (Q and O always are), for
-// calls whose requests have few query tokens.
-template <int DT, int D, int NQ, int NP, int NS, bool STREAM_KV = false>
+// calls whose requests have few query tokens. WRITE_PLAN: the row lists are left
+// in plan_count / plan_rows; a form of its own, since a uniform branch on it cost
+// every other call up to 2% (245 tokens of 64 heads x 128 17.8 -> 18.2 us, 4000
+// of 32 heads x 128 85.7 -> 89.6 with the stores).
+template <int DT, int D, int NQ, int NP, int NS, bool STREAM_KV = false, bool WRITE_PLAN = false>
 __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a) {
   typedef typename B16<DT>::scalar scalar;
   typedef typename B16<DT>::x8 x8;
@@ -559,10 +561,11 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
       }
     }
     block_barrier();
-    if constexpr (D != 512) {
-      if (a.write_plan && head0 == 0) {
-        // The plan as sparse_plan_kernel writes it. These stores only make the
-        // load waits below stricter: vmcnt counts them too.
+    if constexpr (WRITE_PLAN) {
+      if (head0 == 0) {
+        // The plan as sparse_plan_kernel writes it. These stores may still be
+        // in flight at the counted waits of the first steps: vmcnt counts them
+        // too, which makes those waits stricter, never weaker.
         uint32_t* dst = a.plan_rows + (size_t)token * a.list_pad;
         for (int r = tid; r < max(padded, CHUNK); r += NT) dst[r] = n_rows > 0 ? row_list[r] : 0u;
         if (tid == 0) a.plan_count[token] = n_rows;
@@ -583,7 +586,8 @@ __global__ __launch_bounds__((NQ + NP) * 64) void sparse_mla_kernel(SparseArgs a
   // holds the swizzled rows without VGPR staging or ds_write traffic. M0 is
   // set inside the same asm statement; nothing else in this kernel uses M0.
   // Completion is tracked with vmcnt: when a step waits, the only vector
-  // memory loads in flight are the previous fetch's.
+  // memory loads in flight are the previous fetches' (and, early on, the stores
+  // of the debug image or the plan, which only make the waits stricter).
   // With D = 512 one wave load covers exactly one 1 KiB row, so a fetching
   // wave takes FPW consecutive rows whose list entries and addresses are
   // wave-uniform (scalar registers), and the entries are read one step ahead.
@@ -1665,7 +1669,6 @@ static SparseArgs make_args(const SparseMlaParams* p, const void* q, const void*
   a.list_pad = (p->WINDOW + p->TOPK + 255) / 256 * 256;
   a.plan_rows = nullptr;
   a.plan_count = nullptr;
-  a.write_plan = 0;
   a.partials = nullptr;
   const Split split = choose_split(p);
   a.parts = split.parts;
@@ -1782,17 +1785,18 @@ static int after_one_item(const SparseArgs& a, int64_t tiles, hipStream_t stream
 }
 
 template <int DT, int D, int NQ, int NP>
-static int launch_fused(SparseArgs a, hipStream_t stream) {
+static int launch_fused(const SparseArgs& a, hipStream_t stream) {
   const size_t lds = (size_t)a.list_pad * sizeof(uint32_t);
   const int64_t tiles = (int64_t)a.T * (a.H / a.BM);
   static const int cus = device_cus();
-  if (a.plan_rows != nullptr && a.parts == 1 && tiles >= 2 * (int64_t)cus) {
+  const bool leave_plan = a.plan_rows != nullptr && a.parts == 1 && tiles >= 2 * (int64_t)cus;
+  if (leave_plan) {
     // Two items per CU and more, unsplit: the plan stays in the workspace.
     // D = 512, where one workgroup fills a CU: plan kernel, then the persistent
     // kernel over the plan (it removes the per-item start, which outweighs a
     // second kernel), where a KV ring with its row-list ring fits. Smaller D:
     // two or three workgroups of the one-item kernel share a CU and hide each
-    // other's start, and it leaves the plan itself; measured against plan +
+    // other's start, and a form of it leaves the plan itself; measured against plan +
     // persistent (one workgroup per CU / the best of one to three, us): 1403
     // tokens of 32 heads x 256 f16 66 / 112 / 77, 8000 bf16 348 / 655 / 361;
     // 2000 of 64 heads x 256 102 / 142 / 142; of 64 heads x 128 4000 122 / 209
@@ -1806,8 +1810,6 @@ static int launch_fused(SparseArgs a, hipStream_t stream) {
         if (e != hipSuccess) return (int)e;
         return launch_persistent<DT, D, NQ, NP>(a, ring, stream);
       }
-    } else {
-      a.write_plan = 1;
     }
   }
   // One workgroup per item (whole keys, then the parts of split keys): a
@@ -1825,6 +1827,10 @@ static int launch_fused(SparseArgs a, hipStream_t stream) {
                            a);
         return after_one_item<DT, D, NQ, NP>(a, tiles, stream);
       }
+    } else if (leave_plan) {
+      hipLaunchKernelGGL((sparse_mla_kernel<DT, D, NQ, NP, 4, false, true>), dim3(blocks), dim3((NQ + NP) * 64), lds,
+                         stream, a);
+      return (int)hipGetLastError();
     }
     hipLaunchKernelGGL((sparse_mla_kernel<DT, D, NQ, NP, 4>), dim3(blocks), dim3((NQ + NP) * 64), lds, stream, a);
   } else {
@@ -1836,6 +1842,10 @@ static int launch_fused(SparseArgs a, hipStream_t stream) {
                            a);
         return after_one_item<DT, D, NQ, NP>(a, tiles, stream);
       }
+    } else if (leave_plan) {
+      hipLaunchKernelGGL((sparse_mla_kernel<DT, D, NQ, NP, 3, false, true>), dim3(blocks), dim3((NQ + NP) * 64), lds,
+                         stream, a);
+      return (int)hipGetLastError();
     }
     hipLaunchKernelGGL((sparse_mla_kernel<DT, D, NQ, NP, 3>), dim3(blocks), dim3((NQ + NP) * 64), lds, stream, a);
   }

@@ -109,7 +109,7 @@ class Binding:
     contiguity and device in one pass and repeats the pairwise disjointness
     check only when a pointer differs from the last validated call."""
 
-    __slots__ = ("device", "stream", "specs", "params", "params_ref", "nbytes", "workspace", "validated")
+    __slots__ = ("device", "stream", "specs", "params", "params_ref", "nbytes", "own_nbytes", "workspace", "validated")
 
     def __init__(self, device, stream, specs, params, nbytes):
         self.device = device
@@ -118,6 +118,11 @@ class Binding:
         self.params = params
         self.params_ref = ct.pointer(params)
         self.nbytes = nbytes
+        # Of the workspace the call makes itself. Below D = 512 unsplit calls
+        # only leave their row-list plan in it, which nobody reads there.
+        _, rows, entries = plan_layout(params.T, params.WINDOW, params.TOPK)
+        plan_only = nbytes == rows + 4 * params.T * entries
+        self.own_nbytes = 0 if params.D != 512 and plan_only else nbytes
         self.workspace = None
         self.validated = None
 
@@ -262,12 +267,12 @@ def _prepare(
                 and workspace.device == b.device, "workspace must be a contiguous uint8 tensor on the operands' device")
         require(workspace.numel() >= b.nbytes, f"workspace holds {workspace.numel()} bytes, needs {b.nbytes}")
         extra += (("workspace", workspace),)
-    elif b.nbytes:
+    elif b.own_nbytes:
         if torch._C._cuda_isCurrentStreamCapturing():
-            workspace = torch.empty(b.nbytes, dtype=torch.uint8, device=b.device)
+            workspace = torch.empty(b.own_nbytes, dtype=torch.uint8, device=b.device)
         else:
             if b.workspace is None:
-                b.workspace = torch.empty(b.nbytes, dtype=torch.uint8, device=b.device)
+                b.workspace = torch.empty(b.own_nbytes, dtype=torch.uint8, device=b.device)
             workspace = b.workspace
     ws_ptr = None if workspace is None else workspace.data_ptr()
     signature = (*ptrs, ws_ptr, *((name, t.data_ptr(), t.numel()) for name, t in extra))
@@ -320,9 +325,10 @@ def sparse_mla(*args, **kwargs):
     chunks (32 entries of ori_kv row 0 for an empty selection).
 
     Without ``workspace``, each (device, stream, sizes) binding keeps one
-    workspace and reuses it for every call on that stream (calls on one
-    stream run in order); under HIP graph capture the call allocates its own
-    from the graph's pool instead. ``release_bindings()`` frees them.
+    workspace where the call needs one (below D = 512 only to split keys) and
+    reuses it for every call on that stream (calls on one stream run in
+    order); under HIP graph capture the call allocates its own from the
+    graph's pool instead. ``release_bindings()`` frees them.
     """
     _, stream, ptrs, ws_ptr, params_ref, _, out = _prepare(*args, **kwargs)
     _native.check(_native.library().launch_sparse_mla(stream, *ptrs, ws_ptr, params_ref), "launch_sparse_mla")

@@ -43,6 +43,16 @@ def test_plan_and_output_match_the_persistent_kernel(device, d, h, bm, topk, cas
     out = tensors["attention_out"].clone()
     sample = [0, 1, items // 2, items - 1]
     assert_close(out.float().cpu().numpy()[sample], sr.oracle_fp32(data, policy, sample), policy["DTYPE"])
+    for t in (tensors["attention_out"], lse):
+        t.fill_(float("nan"))
+    sparse_mla(*call_args(tensors), **call_kwargs(policy), softmax_lse=lse)  # no plan left, perhaps split keys
+    torch.cuda.synchronize()
+    if items >= 512:
+        assert torch.equal(out, tensors["attention_out"])
+    else:
+        assert_close(tensors["attention_out"].float().cpu().numpy()[sample], sr.oracle_fp32(data, policy, sample),
+                     policy["DTYPE"])
+    sparse_mla(*call_args(tensors), **call_kwargs(policy), parts=1, softmax_lse=lse)
     planned_lse = torch.empty_like(lse)
     kw = call_kwargs(policy)
     sparse_mla_planned(*(tensors[k] for k in ("q", "ori_kv", "cmp_kv", "sinks", "attention_out")),

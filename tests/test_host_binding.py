@@ -69,6 +69,15 @@ def test_binding_holds_the_calls_parameters_and_workspace_size():
     assert b.specs[0][2] is torch.bfloat16 and make(dtype="f16").specs[0][2] is torch.float16
 
 
+def test_a_call_makes_no_workspace_that_only_takes_a_plan():
+    """Below D = 512 an unsplit call reads no plan: it makes no workspace of its
+    own. D = 512 (plan + persistent kernel) and split keys need all of it."""
+    narrow = dict(D=256, H=32, BM=32)
+    for over, own in ((dict(T=1024, **narrow), False), (dict(T=1024), True), (dict(T=16, **narrow), True), (dict(T=16), True)):
+        b = make(**over)
+        assert b.nbytes > 0 and b.own_nbytes == (b.nbytes if own else 0), over
+
+
 def test_binding_cache_is_bounded():
     first = make(stream=1000)
     for k in range(A.MAX_BINDINGS):
