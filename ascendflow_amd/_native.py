@@ -35,6 +35,7 @@ EXPORTS = (
     "workspace_size_sparse_topk_indices_split",
     "launch_attention_target",
     "launch_attention_target_split",
+    "form_attention_target",
     "launch_simple_attention",
     "kernel_config_sparse_mla",
     "kernel_config_attention_target",
@@ -103,6 +104,10 @@ _SIGNATURES = {
     "launch_sparse_topk_indices": ([_P] * 7, ct.c_int),
     "launch_sparse_topk_indices_split": ([_P] * 7 + [ct.c_uint64, _P], ct.c_int),
     "workspace_size_sparse_topk_indices_split": ([ct.POINTER(ct.c_uint64), _P], ct.c_int),
+    "form_attention_target": (
+        [ct.POINTER(ct.c_int64), ct.c_int64, ct.c_int64, ct.POINTER(FaParams), ct.c_int],
+        ct.c_int,
+    ),
     "launch_attention_target": (
         [_P] * 6 + [ct.c_int64, ct.c_int64, ct.POINTER(FaParams)],
         ct.c_int,

@@ -1132,6 +1132,17 @@ extern "C" int launch_attention_target_split(void* stream, const void* Q, const 
   return dispatch_fa(a, plan, workspace, p->dtype, (hipStream_t)stream);
 }
 
+extern "C" int form_attention_target(int64_t form[3], int64_t Sq, int64_t Sk, const FaParams* p, int with_workspace) {
+  if (!form) return AFA_E_NULL;
+  const int status = check_fa(Sq, Sk, p);
+  if (status) return status;
+  const FaPlan plan = choose_fa(make_fa(nullptr, nullptr, nullptr, nullptr, Sq, Sk, p), with_workspace != 0);
+  form[0] = plan.qt ? 1 : 0;
+  form[1] = plan.qt ? 16 * plan.qt : FA_ROWS[plan.form];
+  form[2] = plan.splits;
+  return AFA_OK;
+}
+
 extern "C" int launch_simple_attention(void* stream, const void* Q, const void* K, const void* V,
                                        void* O, void* workspace, int64_t S, int64_t H) {
   (void)workspace;

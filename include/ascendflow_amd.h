@@ -179,6 +179,12 @@ int launch_attention_target_split(void* stream, const void* Q, const void* K, co
                                   void* workspace, uint64_t workspace_bytes, int64_t Sq, int64_t Sk,
                                   const FaParams* params);
 
+/* Which kernel a call of these sizes runs, with and without a workspace (the
+ * launchers choose by the sizes alone): form[0] 0 for the forward kernel, 1 for
+ * the kernel over packed query rows; form[1] its query rows per workgroup;
+ * form[2] the key splits (1: no second kernel). For tests and profiles. */
+int form_attention_target(int64_t form[3], int64_t Sq, int64_t Sk, const FaParams* params, int with_workspace);
+
 /* Teaching attention: examples/flash_attention/simple.py:60-141.
  *   Q [H,S,128] f16, K/V [H,128,128] f16, O [H,S,128] f16 (written);
  * softmax(QK^T / sqrt(128)) normalised before the f16 cast of P. */

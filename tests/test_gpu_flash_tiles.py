@@ -8,6 +8,7 @@ import pytest
 
 from oracle.attention import inputs
 from tests.test_gpu_flash import assert_contract, online_rows, run_fa
+from tests.test_gpu_flash_split import form_of
 
 pytestmark = pytest.mark.gpu
 
@@ -32,6 +33,7 @@ pytestmark = pytest.mark.gpu
 )
 def test_tiles_match_the_reference_contract(device, b, hq, hkv, sq, sk, dtype, causal, case):
     print(f"\n[fa tiles] b={b} hq={hq} hkv={hkv} sq={sq} sk={sk} {dtype} causal={causal} case={case}", flush=True)
+    assert form_of(b, hq, hkv, sq, sk, causal) == (0, 64 if b < 40 else 128, 1)
     data = inputs(b, hq, hkv, sq, sk, dtype, scale=0.5, case=case)
     actual = run_fa(data, dtype, causal, device)
     rows = np.array(sorted({min(r, sq - 1) for r in (0, 15, 16, 62, 63, 64, 127, 128, sq // 2, sq - 1)}))
