@@ -33,6 +33,7 @@ EXPORTS = (
     "launch_sparse_topk_indices",
     "launch_sparse_topk_indices_split",
     "workspace_size_sparse_topk_indices_split",
+    "form_sparse_topk_indices",
     "launch_attention_target",
     "launch_attention_target_split",
     "form_attention_target",
@@ -104,6 +105,7 @@ _SIGNATURES = {
     "launch_sparse_topk_indices": ([_P] * 7, ct.c_int),
     "launch_sparse_topk_indices_split": ([_P] * 7 + [ct.c_uint64, _P], ct.c_int),
     "workspace_size_sparse_topk_indices_split": ([ct.POINTER(ct.c_uint64), _P], ct.c_int),
+    "form_sparse_topk_indices": ([ct.POINTER(ct.c_int64), _P, ct.c_int], ct.c_int),
     "form_attention_target": (
         [ct.POINTER(ct.c_int64), ct.c_int64, ct.c_int64, ct.POINTER(FaParams), ct.c_int],
         ct.c_int,

@@ -1424,3 +1424,14 @@ extern "C" int launch_sparse_topk_indices_split(void* stream, const float* score
   return launch_topk((hipStream_t)stream, scores, cu_seqlens_q, seqused_cmp_kv, cmp_residual_kv, cmp_sparse_indices,
                      workspace, params, plan);
 }
+
+extern "C" int form_sparse_topk_indices(int64_t form[3], const SparseTopkParams* params, int with_workspace) {
+  if (!form) return AFA_E_NULL;
+  const int status = check_topk(params);
+  if (status) return status;
+  const TopkPlan plan = choose_topk(params, with_workspace != 0);
+  form[0] = plan.form;
+  form[1] = plan.form == TK_FORM_ROW ? plan.threads : plan.form == TK_FORM_SPLIT ? plan.segments : 0;
+  form[2] = plan.form == TK_FORM_ROW ? plan.items : plan.form == TK_FORM_SPLIT ? plan.tokens : 0;
+  return AFA_OK;
+}

@@ -296,6 +296,12 @@ int launch_sparse_topk_indices_split(void* stream, const float* scores, const in
                                      int32_t* cmp_sparse_indices, void* workspace, uint64_t workspace_bytes,
                                      const SparseTopkParams* params);
 
+/* Which form a call of these sizes runs, with and without a workspace: form[0]
+ * 0 rows in registers (form[1] threads, form[2] positions per thread), 1 split
+ * rows (form[1] segments per row, form[2] tokens per pair of launches), 2 the
+ * filter pass, 3 the streaming passes. For tests and profiles. */
+int form_sparse_topk_indices(int64_t form[3], const SparseTopkParams* params, int with_workspace);
+
 /* Measurement helpers (no reference kernel; the reference sweeps a >= 4x L2
  * buffer before each timed launch, benchmarks/cache.py:13-92 and
  * benchmarks/cache_sweep.py:15-32). Reads `bytes` of `buffer` through the

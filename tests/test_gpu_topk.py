@@ -75,8 +75,9 @@ def test_ties_spanning_many_chunks_match_the_oracle(device, c):
     """Few distinct values: the threshold key is shared by thousands of
     positions, so the equal keys taken are spread over the whole row (and
     more than the filter kernel's buffer reach the estimate). The widths run
-    up to the filter kernel's 256K-position limit and past it, where the
-    streaming form takes over."""
+    up to the filter kernel's 256K positions and past them; the two widest are
+    split rows (test_gpu_topk_rows.py has such widths without a workspace, in
+    the filter and the streaming form)."""
     rng = np.random.default_rng(c)
     cu = np.array([0, 20, 40], np.int32)
     seq_cmp = np.array([c, c // 2], np.int32)

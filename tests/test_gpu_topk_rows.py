@@ -1,9 +1,11 @@
 """The register form of the top-k selection (sparse_topk_row) and its split form,
 bit-exact against the oracle at the edges of their sizes: rows either side of
-each register size, both workgroup sizes, TOPK either side of the entries the
-kernel holds, segment edges; and calls of many tokens, which the streaming
-form serves (its linear histograms and their radix fallback). Scores: normal, heavy ties, constant, infinities and NaN, masked
-with -inf, one outlier that spans the histogram."""
+each register size, both workgroup sizes, TOPK up to and past what these forms
+take, segment edges, calls of more tokens than one pair of launches; the filter
+form (its linear histograms and their radix fallback) and the streaming one, also
+without a workspace. Every case states the form that the sizes choose and checks
+it. Scores: normal, heavy ties, constant, infinities and NaN, masked with -inf,
+one outlier that spans the histogram."""
 
 import ctypes as ct
 
@@ -11,6 +13,9 @@ import numpy as np
 import pytest
 import torch
 
+from ascendflow_amd import _native
+from ascendflow_amd._tensors import stream_handle
+from ascendflow_amd.sparse_attention.indexer import SparseTopkParams
 from oracle import topk_reference as tr
 
 
@@ -36,10 +41,22 @@ def scores_of(kind, rng, t, c):
     return s
 
 
-def check(device, t, c, topk, kind, ratio=1, short=True, seed=0):
+ROW, SPLIT, FILTER, STREAM = range(4)
+
+
+def form_of(t, c, topk, ratio=1, workspace=True):
+    """(form, threads or segments, positions per thread or tokens per pair of launches) of a call."""
+    params = SparseTopkParams(3, t, topk, ratio, c)
+    form = (ct.c_int64 * 3)()
+    assert _native.library().form_sparse_topk_indices(form, ct.byref(params), int(workspace)) == 0
+    return tuple(form)
+
+
+def check(device, t, c, topk, kind, form, ratio=1, short=True, seed=0, workspace=True):
     from ascendflow_amd.sparse_attention import sparse_topk_indices
 
-    print(f"\n[topk rows] T={t} C={c} TOPK={topk} {kind} R={ratio}", flush=True)
+    print(f"\n[topk rows] T={t} C={c} TOPK={topk} {kind} R={ratio} form={form}", flush=True)
+    assert form_of(t, c, topk, ratio, workspace)[:len(form)] == form, "the call runs another form than this case is for"
     rng = np.random.default_rng(seed + t * 7 + c)
     scores = scores_of(kind, rng, t, c)
     # Three requests: one over the whole row, one over part of it, one empty.
@@ -50,7 +67,14 @@ def check(device, t, c, topk, kind, ratio=1, short=True, seed=0):
     to = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=device)
     buffer = torch.full((t * topk + 64,), 7, dtype=torch.int32, device=device)
     out = buffer[: t * topk].view(t, 1, topk)
-    sparse_topk_indices(to(scores), to(cu), to(seq_cmp), to(residual), TOPK=topk, RATIO=ratio, out=out)
+    tensors = [to(a) for a in (scores, cu, seq_cmp, residual)]
+    if workspace:
+        sparse_topk_indices(*tensors, TOPK=topk, RATIO=ratio, out=out)
+    else:
+        status = _native.library().launch_sparse_topk_indices(
+            stream_handle(device), *(x.data_ptr() for x in tensors), out.data_ptr(),
+            ct.byref(SparseTopkParams(3, t, topk, ratio, c)))
+        assert status == 0
     torch.cuda.synchronize()
     assert torch.all(buffer[t * topk:] == 7), "write past the output"
     np.testing.assert_array_equal(out.cpu().numpy(), tr.topk_indices(scores, cu, seq_cmp, residual, topk, ratio))
@@ -58,37 +82,69 @@ def check(device, t, c, topk, kind, ratio=1, short=True, seed=0):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["normal", "ties", "constant", "special", "masked", "lowest", "outlier", "tiny"])
-@pytest.mark.parametrize("t,c,topk", [(3, 4096, 512), (3, 8193, 512), (258, 700, 96), (4, 70001, 512), (2049, 1501, 96)])
-def test_score_distributions(device, t, c, topk, kind):
-    check(device, t, c, topk, kind, ratio=2)
+@pytest.mark.parametrize(
+    "t,c,topk,form",
+    [(3, 4096, 512, (ROW, 1024, 4)), (3, 8193, 512, (ROW, 1024, 16)), (258, 700, 96, (ROW, 512, 8)),
+     (4, 70001, 512, (FILTER,)), (4, 90001, 512, (SPLIT, 6)), (2049, 1501, 96, (FILTER,))],
+)
+def test_score_distributions(device, t, c, topk, kind, form):
+    check(device, t, c, topk, kind, form, ratio=2)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize(
-    "t,c,topk",
-    [(2, 1, 1), (2, 63, 64), (3, 2047, 2046), (3, 2048, 2040), (3, 2049, 400), (3, 4095, 700), (3, 4097, 768),
-     (2, 8192, 1024), (2, 16383, 1500), (2, 16384, 1), (2, 16385, 512), (2, 32768, 1536), (257, 4096, 300),
-     (257, 4099, 512), (258, 8191, 512), (259, 16385, 512), (2049, 300, 96), (2049, 301, 96), (1030, 17000, 512)],
+    "t,c,topk,form",
+    [(2, 1, 1, (ROW, 1024, 4)), (2, 63, 64, (ROW, 1024, 4)), (3, 1500, 1408, (ROW, 1024, 4)), (3, 2047, 2046, (FILTER,)),
+     (3, 2048, 2040, (FILTER,)), (3, 2049, 400, (ROW, 1024, 4)), (3, 4095, 700, (ROW, 1024, 4)),
+     (3, 4097, 768, (ROW, 1024, 8)), (2, 8192, 1024, (ROW, 1024, 8)), (2, 16383, 1408, (ROW, 1024, 16)),
+     (2, 16383, 1500, (FILTER,)), (2, 16384, 1, (ROW, 1024, 16)), (2, 16385, 512, (ROW, 1024, 32)),
+     (2, 32768, 1408, (ROW, 1024, 32)), (2, 32768, 1536, (FILTER,)), (2, 32769, 512, (FILTER,)),
+     (256, 4097, 300, (ROW, 1024, 8)), (257, 4096, 300, (ROW, 512, 8)), (257, 4099, 512, (ROW, 512, 16)),
+     (258, 8191, 512, (ROW, 512, 16)), (257, 8193, 1408, (ROW, 512, 32)), (259, 16385, 512, (ROW, 512, 64)),
+     (1024, 300, 96, (ROW, 512, 8)), (1025, 300, 96, (FILTER,)), (2049, 300, 96, (FILTER,)), (2049, 301, 96, (FILTER,)),
+     (1024, 17000, 512, (ROW, 512, 64)), (1030, 17000, 512, (FILTER,))],
 )
-def test_row_sizes(device, t, c, topk):
-    check(device, t, c, topk, "normal", ratio=1 + c % 2)
+def test_row_sizes(device, t, c, topk, form):
+    check(device, t, c, topk, "normal", form, ratio=1 + c % 2)
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize(
-    "t,c,topk,kind",
-    [(2, 65537, 512, "normal"), (2, 81920, 1, "normal"), (3, 98303, 1024, "ties"), (2, 131073, 2047, "special"),
-     (1, 163840, 3000, "normal"), (2, 262145, 512, "ties"), (1, 300003, 1700, "normal"), (1, 524289, 512, "outlier"),
-     (2, 65600, 16384, "normal")],
+    "t,c,topk,kind,form",
+    [(2, 65537, 512, "normal", (FILTER,)), (2, 81920, 1, "normal", (FILTER,)), (2, 81921, 1, "normal", (SPLIT, 6)),
+     (3, 98303, 1024, "ties", (SPLIT, 6)), (3, 98305, 1408, "special", (SPLIT, 7)), (2, 131073, 2047, "special", (FILTER,)),
+     (1, 163840, 3000, "normal", (FILTER,)), (3, 262144, 1408, "normal", (SPLIT, 16)), (2, 262145, 512, "ties", (SPLIT, 17)),
+     (2, 262145, 1924, "normal", (SPLIT, 17)), (1, 300003, 1700, "normal", (SPLIT, 19)),
+     (1, 524289, 512, "outlier", (SPLIT, 33)), (2, 65600, 16384, "normal", (FILTER,))],
 )
-def test_split_rows(device, t, c, topk, kind):
-    check(device, t, c, topk, kind, ratio=2)
+def test_split_rows(device, t, c, topk, kind, form):
+    check(device, t, c, topk, kind, form, ratio=2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["normal", "ties", "special"])
+def test_split_rows_in_several_pairs_of_launches(device, kind):
+    """One token more than a pair of launches has workspace for."""
+    form = form_of(260, 262145, 1900)
+    assert form == (SPLIT, 17, 259)
+    check(device, 260, 262145, 1900, kind, form)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "t,c,topk,kind,form,workspace",
+    [(2, 262145, 1925, "normal", (STREAM,), True),  # more entries than the merge takes
+     (3, 262145, 512, "special", (STREAM,), False), (2, 300001, 700, "ties", (STREAM,), False),
+     (1, 524289, 512, "outlier", (STREAM,), False), (3, 262144, 512, "normal", (FILTER,), False),
+     (3, 262144, 1024, "ties", (FILTER,), False), (3, 200001, 512, "special", (FILTER,), False)],
+)
+def test_rows_that_are_not_split(device, t, c, topk, kind, form, workspace):
+    """The streaming form, and the filter form up to its 256K positions: the
+    entry without a workspace, and TOPK beyond the merge's."""
+    check(device, t, c, topk, kind, form, ratio=2, workspace=workspace)
 
 
 def test_split_entry_refuses_a_small_workspace():
-    from ascendflow_amd import _native
-    from ascendflow_amd.sparse_attention.indexer import SparseTopkParams
-
     lib = _native.library()
     need = ct.c_uint64(0)
     params = SparseTopkParams(1, 4, 512, 2, 524288)
