@@ -43,7 +43,14 @@ def test_wrong_operands_are_refused_by_name(device, entry):
                 continue  # the sizes come from these two: another size is another valid call
             with pytest.raises(ValueError, match=name if i else ".*"):
                 call([*tensors[:i], bad, *tensors[i + 1:]])
-    if entry != "topk":
+    if entry == "topk":
+        indices_in_scores = tensors[0].view(torch.int32).view(-1)[16:32].view(2, 1, 8)
+        cu_in_indices = tensors[4].view(-1)[14:]
+        cu_in_indices.copy_(tensors[1])
+        overlapping = [tensors[:4] + [indices_in_scores], [tensors[0], cu_in_indices, *tensors[2:]]]
+    else:
+        overlapping = [[tensors[output], *tensors[1:]], [tensors[0], tensors[output], *tensors[2:]]]
+    for operands in overlapping:
         with pytest.raises(ValueError, match="overlap"):
-            call([tensors[output], *tensors[1:]])
+            call(operands)
     torch.cuda.synchronize()
