@@ -802,8 +802,9 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaSplitArgs args) {
 // 256-byte rows (straight from the accumulators a store instruction writes 16
 // pieces of 32 bytes). Two workgroups share a CU (80 KiB of LDS each). Two row
 // tiles per wave, which read each fragment for twice the MFMAs, measured the
-// same. Measured call, one tile per workgroup -> this: H32 S8192 67.1 -> 36.1
-// us (3.8 TB/s), H64 S8192 132.8 -> 61.0 (4.4 TB/s), H64 S2048 29.1 -> 17.6.
+// same. GPU time of a call, one tile per workgroup -> this (us): H4 S128 5.37 ->
+// 5.23, H32 S1024 11.4 -> 7.95, H64 S2048 28.3 -> 17.8, H32 S8192 49.7 -> 32.9
+// (4.1 TB/s), H64 S8192 125 -> 62.1 (4.3 TB/s).
 __global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16* Qp, const _Float16* Kp,
                                                                   const _Float16* Vp, _Float16* Op, int64_t S,
                                                                   int32_t groups, int32_t steps) {
@@ -831,13 +832,16 @@ __global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16
       for (int j = 0; j < D / 32; ++j) qf[j] = *(const f16x8*)(Q + (row + i16) * D + 32 * j + 8 * g);
     }
   };
-  load_q(0);
   for (int flat = tid; flat < SK * (D / 8); flat += 256) {
     const int r = flat / (D / 8), u = flat % (D / 8);
     const int off = r * ROW_BYTES + (swz(r, u) << 4);
     *(u32x4*)(&k_lds[off]) = *(const u32x4*)(K + r * D + u * 8);
     *(u32x4*)(&v_lds[off]) = *(const u32x4*)(V + r * D + u * 8);
   }
+  // After K and V: loads return in order, so Q's first, in pieces of 64 bytes,
+  // would hold up the whole workgroup's tile (H4 S128 5.62 us, so 5.23; H32 S1024
+  // 8.8, so 7.95).
+  load_q(0);
   __syncthreads();
 
   const int ra = sigma(i16);
