@@ -33,6 +33,7 @@ struct FaArgs {
   void* o;
   int64_t Sq, Sk;
   int32_t B, HQ, HKV, causal;
+  int32_t level_order;  // causal forward kernel: the longest tiles of all heads first
   float scale;
 };
 
@@ -95,12 +96,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_forward_kernel(Fa
   const int g = lane >> 4, i16 = lane & 15;
   const int64_t q_tiles = (a.Sq + BQ - 1) / BQ;
   int64_t qtile, bh;
-  if (a.causal) {
+  if (a.level_order) {
     // Tiles of all heads from the longest down. The dispatcher deals workgroups
     // to an XCD's shader engines in turn, so with a head's tiles in a row and
     // an even number of them, engine 0 got the long ones of every head (B2
-    // HQ32 S1987 126 -> 84 us; B1 HQ32 S4096 211 -> 147; S8192 564 -> 549). Heads that share a
-    // KV head stay on one XCD (blocks go to XCD blockIdx % 8).
+    // HQ32 HKV8 S1987 126 -> 80 us with this and 128-row tiles; 256-row tiles, B1
+    // HQ32 S4096 211 -> 147). Heads that share a KV head stay on one XCD (blocks
+    // go to XCD blockIdx % 8). All heads' keys are read again at every level:
+    // only while they stay in the Infinity Cache (FA_LEVEL_BYTES).
     const uint32_t heads = (uint32_t)a.B * (uint32_t)a.HQ;
     const uint32_t level = blockIdx.x / heads, i = blockIdx.x % heads;
     qtile = q_tiles - 1 - level;
@@ -108,6 +111,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void fa_forward_kernel(Fa
   } else {
     const uint32_t logical = xcd_contiguous(blockIdx.x, gridDim.x);
     qtile = (int64_t)(logical % q_tiles);
+    if (a.causal) qtile = q_tiles - 1 - qtile;
     bh = logical / q_tiles;
   }
   const int head = (int)(bh % a.HQ), batch = (int)(bh / a.HQ);
@@ -929,6 +933,12 @@ namespace {
 constexpr int FD_MAX_SPLITS = 64;  // fa_merge_kernel keeps two splits per thread of a row
 constexpr int64_t FA_CUS = 256;
 constexpr int64_t FD_STREAM_BYTES = int64_t(128) << 20;
+// K and V of a causal call up to which the forward kernel takes the tiles of all
+// heads by length; beyond, a head's tiles follow each other and read its keys
+// from the L2. 128-row tiles by length / by head (us): 142 MiB 174 / 176, 219
+// 372 / 380, 255 525 / 513, 266 388 / 364, 321 341 / 319, 445 849 / 711, 593 1017
+// / 732 (256-row tiles by head: 771).
+constexpr int64_t FA_LEVEL_BYTES = int64_t(240) << 20;
 
 template <int DT, int NW, int QT>
 int launch_forward(const FaArgs& a, hipStream_t s) {
@@ -1090,6 +1100,7 @@ FaArgs make_fa(const void* Q, const void* K, const void* V, void* O, int64_t Sq,
   a.HQ = p->HQ;
   a.HKV = p->HKV;
   a.causal = p->causal ? 1 : 0;
+  a.level_order = a.causal && 2 * 256 * (int64_t)p->B * p->HKV * std::min(Sq, Sk) <= FA_LEVEL_BYTES;
   a.scale = p->scale;
   return a;
 }

@@ -1,13 +1,16 @@
 """The forward flash-attention kernel in tiles of 128 and 64 query rows (four
 waves, two slots per tensor in the KV ring): one, two and more key chunks, a
 ragged last one, tiles either side of their rows, causal and grouped heads,
-against the online oracle at the contract tolerance of test_gpu_flash.py."""
+against the online oracle at the contract tolerance of test_gpu_flash.py; and
+causal calls whose keys fit the Infinity Cache (tiles of all heads by length)
+and do not (tiles head by head)."""
 
 import numpy as np
 import pytest
+import torch
 
 from oracle.attention import inputs
-from tests.test_gpu_flash import assert_contract, online_rows, run_fa
+from tests.test_gpu_flash import TORCH, assert_contract, online_rows, run_fa
 from tests.test_gpu_flash_split import form_of
 
 pytestmark = pytest.mark.gpu
@@ -41,3 +44,27 @@ def test_tiles_match_the_reference_contract(device, b, hq, hkv, sq, sk, dtype, c
     assert np.isfinite(actual).all()
     expected = online_rows(data["q"][few], data["k"][few], data["v"][few], rows, dtype, causal, 64)
     assert_contract(actual[few][:, :, rows], expected, dtype)
+
+
+@pytest.mark.parametrize("b,hq,hkv,sq,sk,dtype", [
+    (60, 64, 64, 128, 200, "bf16"),  # 240 MiB of visible keys and values: by length
+    (60, 64, 64, 129, 129, "f16"),   # 242 MiB, heads a multiple of the 8 XCDs: head by head
+    (75, 27, 27, 257, 300, "bf16"),  # 254 MiB, heads not
+])
+def test_causal_tile_orders(device, b, hq, hkv, sq, sk, dtype):
+    from ascendflow_amd.flash_attention import attention_target
+
+    print(f"\n[fa order] b={b} hq={hq} hkv={hkv} sq={sq} sk={sk} {dtype}", flush=True)
+    assert form_of(b, hq, hkv, sq, sk, True)[0] == 0
+    torch.manual_seed(sq)
+    q, k, v = (torch.randn((b, h, s, 128), device=device, dtype=TORCH[dtype]) * 0.5
+               for h, s in ((hq, sq), (hkv, sk), (hkv, sk)))
+    o = torch.full_like(q, float("nan"))
+    attention_target(q, k, v, o, sq, sk, B=b, HQ=hq, HKV=hkv, D=128, DTYPE=dtype, SCALE=128**-0.5, CAUSAL=True)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(o).all())
+    batches, heads = [0, b // 2, b - 1], [0, 1, hq // 2, hq - 1]
+    pick = lambda t: t[batches][:, heads].float().cpu().numpy()
+    rows = np.array(sorted({0, 63, 64, 127, sq - 2, sq - 1}))
+    expected = online_rows(pick(q), pick(k), pick(v), rows, dtype, True, 64)
+    assert_contract(pick(o)[:, :, rows], expected, dtype)
