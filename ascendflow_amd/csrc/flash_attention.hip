@@ -972,7 +972,11 @@ struct FaPlan {
 // workspace size depends on the sizes alone:
 //  - forward kernel: per 64-key chunk ALONE while a CU runs one workgroup of it
 //    (its longest tile then sets the time) and FULL while it runs all that
-//    fit; FORWARD_START for a workgroup's Q, first loads and output;
+//    fit; FORWARD_START for a workgroup's Q, first loads and output; among its
+//    tiles also PAIR_START for 128-row ones, two to a CU, that at most three
+//    chunks follow (256 / 128 / 64 rows: B4 HQ64 S148 15.0 / 16.8 / 18.3; B8 HQ64 S156
+//    27.4 / 29.9 / 26.3; B21 HQ32 Sq139 Sk101 30.9 / 33.6 / 28.2; causal B31 HQ32 S146
+//    49.8 / 43.6 / 36.3);
 //  - split kernel, one workgroup per CU: a step of four 32-key tiles costs the
 //    larger of SPLIT_STEP[qt] (the latency of 64 KiB of loads, then the waves'
 //    own chain of MFMAs and softmax) and KV_STEP, its 64 KiB when all CUs load
@@ -990,7 +994,7 @@ struct FaPlan {
 FaPlan choose_fa(const FaArgs& a, bool with_splits) {
   constexpr int PER_CU[FA_FORMS] = {1, 2, 2};
   constexpr double ALONE[FA_FORMS] = {1.7, 1.25, 0.95}, FULL[FA_FORMS] = {1.8, 1.85, 1.3};
-  constexpr double FORWARD_START[FA_FORMS] = {8.0, 6.5, 5.5};
+  constexpr double FORWARD_START[FA_FORMS] = {8.0, 6.5, 5.5}, PAIR_START = 2.5;
   constexpr double KV_STEP = 2.4, SPLIT_START = 8.0, ROUND = 3.0, ROUND_QT = 1.6, MERGE = 3.0, MERGE_SPLIT = 0.12;
   constexpr double SPLIT_STEP[FD_MAX_QT + 1] = {0, 1.4, 1.55, 2.0, 2.45};
   const int64_t group = a.HQ / a.HKV, kv_heads = (int64_t)a.B * a.HKV, rows = group * a.Sq;
@@ -998,7 +1002,7 @@ FaPlan choose_fa(const FaArgs& a, bool with_splits) {
   // Mean tile length over the longest, with n row tiles per head.
   auto mean = [&](int64_t n) { return a.causal && n > 1 ? 0.5 * (1 + 1.0 / n) : 1.0; };
   FaPlan plan{0, 1, 0, 0};
-  double best = 0;
+  double best = 0, best_pair = 0;  // the cheapest tiles without and with PAIR_START
   for (int form = 0; form < FA_FORMS; ++form) {
     const int64_t tiles = (a.Sq + FA_ROWS[form] - 1) / FA_ROWS[form], blocks = tiles * a.B * a.HQ;
     const double chunks = std::ceil(keys / 64.0), slots = (double)FA_CUS * PER_CU[form];
@@ -1006,10 +1010,12 @@ FaPlan choose_fa(const FaArgs& a, bool with_splits) {
                         std::max(chunks * ALONE[form],
                                  (a.causal ? blocks / slots : std::ceil(blocks / slots)) * mean(tiles) * chunks * FULL[form] *
                                      std::min(1.0, std::max(blocks / slots, 1.0 / PER_CU[form])));
-    if (form == 0 || cost < best) {
-      best = cost;
+    const double with_pair = cost + (form == 1 && blocks > FA_CUS && chunks <= 3 ? PAIR_START : 0.0);
+    if (form == 0 || with_pair < best_pair) {
+      best_pair = with_pair;
       plan.form = form;
     }
+    best = form == 0 ? cost : std::min(best, cost);
   }
   for (int qt = 1; qt <= FD_MAX_QT; ++qt) {
     const int64_t row_tiles = (rows + 16 * qt - 1) / (16 * qt);

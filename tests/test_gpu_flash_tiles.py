@@ -17,26 +17,30 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize(
-    "b,hq,hkv,sq,sk,dtype,causal,case",
+    "b,hq,hkv,sq,sk,dtype,causal,case,tile",
     [
-        # 64-row tiles (small grids)
-        (1, 8, 8, 64, 1, "f16", False, "standard"),
-        (2, 8, 2, 65, 64, "bf16", False, "standard"),
-        (2, 8, 2, 129, 65, "f16", False, "sharp"),
-        (1, 2, 2, 63, 191, "bf16", True, "standard"),
-        (1, 4, 1, 700, 300, "bf16", True, "sharp"),
-        (2, 8, 2, 300, 300, "f16", True, "standard"),
-        # 128-row tiles (more heads than two rounds of 64-row tiles)
-        (48, 8, 8, 257, 64, "bf16", True, "standard"),
-        (40, 16, 16, 129, 65, "f16", False, "standard"),
-        (40, 16, 4, 127, 128, "bf16", False, "sharp"),
-        (48, 8, 8, 120, 193, "f16", False, "standard"),
-        (64, 8, 8, 129, 129, "bf16", True, "standard"),
+        # 64-row tiles: small grids, and short keys on large ones
+        (1, 8, 8, 64, 1, "f16", False, "standard", 64),
+        (2, 8, 2, 65, 64, "bf16", False, "standard", 64),
+        (2, 8, 2, 129, 65, "f16", False, "sharp", 64),
+        (1, 2, 2, 63, 191, "bf16", True, "standard", 64),
+        (1, 4, 1, 700, 300, "bf16", True, "sharp", 64),
+        (2, 8, 2, 300, 300, "f16", True, "standard", 64),
+        (48, 8, 8, 257, 64, "bf16", True, "standard", 64),
+        (40, 16, 16, 129, 65, "f16", False, "standard", 64),
+        (40, 16, 4, 127, 128, "bf16", False, "sharp", 64),
+        (64, 8, 8, 129, 129, "bf16", True, "standard", 64),
+        # 128-row tiles
+        (48, 8, 8, 120, 193, "f16", False, "standard", 128),
+        (40, 16, 4, 127, 256, "bf16", False, "sharp", 128),
+        (64, 8, 8, 129, 193, "f16", False, "standard", 128),
+        (48, 8, 8, 257, 257, "bf16", True, "standard", 128),
+        (12, 32, 32, 257, 300, "f16", True, "sharp", 128),
     ],
 )
-def test_tiles_match_the_reference_contract(device, b, hq, hkv, sq, sk, dtype, causal, case):
+def test_tiles_match_the_reference_contract(device, b, hq, hkv, sq, sk, dtype, causal, case, tile):
     print(f"\n[fa tiles] b={b} hq={hq} hkv={hkv} sq={sq} sk={sk} {dtype} causal={causal} case={case}", flush=True)
-    assert form_of(b, hq, hkv, sq, sk, causal) == (0, 64 if b < 40 else 128, 1)
+    assert form_of(b, hq, hkv, sq, sk, causal) == (0, tile, 1)
     data = inputs(b, hq, hkv, sq, sk, dtype, scale=0.5, case=case)
     actual = run_fa(data, dtype, causal, device)
     rows = np.array(sorted({min(r, sq - 1) for r in (0, 15, 16, 62, 63, 64, 127, 128, sq // 2, sq - 1)}))
