@@ -1258,20 +1258,22 @@ constexpr int64_t TK_SPLIT_BYTES = int64_t(64) << 20;  // workspace of a call, a
 // 45 / 74, 31 / 45, 24 / 22, 20 / 17; 1000 of 20K 0.72x, 0.72x, 1.15x, 1.25x, with TOPK 256
 // 0.98x, 0.98x, 1.07x, 1.34x; 2000 of 16K 40 / 54, 30 / 32, 25 / 23, 24 / 23, 3000 0.82x,
 // 1.00x, 1.10x, 1.11x, 5000 0.86x, 1.08x, 1.18x, 1.20x, with TOPK 1024
-// 0.84x, 0.98x, 0.96x, 0.87x; 2000 of 8K 0.79x, 0.92x, 0.90x, 0.79x; of 700 with TOPK
+// 0.84x, 0.98x, 0.96x, 0.87x; 1300 of 16K with TOPK 256 0.93x, 0.93x, 1.04x, 0.95x, 2000
+// 0.93x, 1.05x, 1.14x, 1.05x; 2000 of 8K 0.79x, 0.92x, 0.90x, 0.79x; of 700 with TOPK
 // 256 0.91x, 1.16x.
 // Split rows, 64 tokens: of 66K 20.2 / 22.0, 17.1 / 16.0, 16.5 / 12.6; of 100K 22.5 / 28.6,
-// 17 / 19, 16 / 14; of 256K 36 / 98, 25 / 54, 19.3 / 21.1, 17.8 / 15.2; 128 tokens: of 128K 34.7
-// / 33.6; of 256K 58 / 99, 37 / 56, 28 / 22. Candidates past one segment and up to about
-// 40K lose 1 to 5 us to the second launch; up to one segment there is nothing to merge
-// (11.5 / 11.8).
+// 17 / 19, 16 / 14; of 256K 36 / 98, 25 / 54, 19.3 / 21.1, 17.8 / 15.2; 96 tokens: of 181K
+// 0.93x, 1.03x, 1.16x, of 215K 0.65x, 0.97x, 1.15x; 128 tokens: of 128K 34.7 / 33.6; of
+// 200K 48.7 / 47.8, 32.9 / 29.9, 26.3 / 20.6; of 256K 58 / 99, 37 / 56, 28 / 22.
+// Candidates past one segment and up to about 40K lose 1 to 5 us to the second
+// launch; up to one segment there is nothing to merge (11.5 / 11.8).
 static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
   TopkPlan plan{};
   const int64_t C = p->C, T = p->T;
   const bool fits = p->TOPK <= 1408;  // entries, whatever the candidates (see the bound)
   const int64_t most = C > 24576   ? 1024
                        : C > 16384 ? (p->TOPK > 256 ? 1024 : 512)
-                       : C > 8192  ? (p->TOPK > 512 ? 5120 : p->TOPK > 256 ? 3072 : 2048)
+                       : C > 8192  ? (p->TOPK > 512 ? 5120 : p->TOPK > 256 ? 3072 : 1300)
                        : C > 1024  ? 2048
                                    : 1024;
   if (C <= 32768 && T <= most && fits) {
@@ -1286,7 +1288,7 @@ static TopkPlan choose_topk(const SparseTopkParams* p, bool with_workspace) {
   }
   const int64_t segments = (C + TK_SEGMENT_SIZE - 1) / TK_SEGMENT_SIZE;
   const int64_t keep = (std::min<int64_t>(p->TOPK, TK_SEGMENT_SIZE) + 3) / 4 * 4;
-  const bool few = T <= 64 || (segments >= 12 && T * segments <= TK_SPLIT_WORKGROUPS);
+  const bool few = T <= 64 || (segments >= (T <= 96 ? 13 : 15) && T * segments <= TK_SPLIT_WORKGROUPS);
   if (with_workspace && segments * keep <= TK_MERGE_MAX &&
       (C > TK_FILTER_MAX_C || (segments >= 6 && few && fits))) {
     plan.form = TK_FORM_SPLIT;
