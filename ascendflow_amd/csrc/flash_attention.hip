@@ -806,14 +806,21 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(FaSplitArgs args) {
 // 256-byte rows (straight from the accumulators a store instruction writes 16
 // pieces of 32 bytes). Two workgroups share a CU (80 KiB of LDS each). Two row
 // tiles per wave, which read each fragment for twice the MFMAs, measured the
-// same. GPU time of a call, one tile per workgroup -> this (us): H4 S128 5.37 ->
-// 5.23, H32 S1024 11.4 -> 7.95, H64 S2048 28.3 -> 17.8, H32 S8192 49.7 -> 32.9
-// (4.1 TB/s), H64 S8192 125 -> 62.1 (4.3 TB/s).
+// same. ONE: one tile per workgroup, a kernel of its own whose Q loads follow K's
+// and V's: loads return in order, and Q's, in pieces of 64 bytes, would hold up
+// the tile that all waves wait for (H4 S128 4.87 -> 4.44 us, H16 S1024 7.17 ->
+// 6.90); over many tiles Q, which comes from HBM, goes first (H32 S8192 38.2, after
+// them 39.4). GPU time of a call over inputs that no cache holds, one tile per
+// workgroup with stores from the accumulators -> this (us): H4 S128 4.62 -> 4.44, H32
+// S1024 11.8 -> 11.0, H64 S2048 37.2 -> 22.5, H32 S8192 65.0 -> 38.3 (3.5 TB/s), H64
+// S8192 128 -> 64 (4.2 TB/s).
+template <bool ONE>
 __global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16* Qp, const _Float16* Kp,
                                                                   const _Float16* Vp, _Float16* Op, int64_t S,
-                                                                  int32_t groups, int32_t steps) {
+                                                                  int32_t groups, int32_t tiles) {
   typedef B16<DT_F16> ops;
   constexpr int D = 128, SK = 128, ROW_BYTES = D * 2, KT = SK / 16, ROWS = 16;
+  const int steps = ONE ? 1 : tiles;
   __shared__ __attribute__((aligned(16))) uint8_t k_lds[SK * ROW_BYTES];
   __shared__ __attribute__((aligned(16))) uint8_t v_lds[SK * ROW_BYTES];
   __shared__ __attribute__((aligned(16))) uint8_t o_lds[4][16 * ROW_BYTES];
@@ -836,16 +843,14 @@ __global__ __launch_bounds__(256, 2) void simple_attention_kernel(const _Float16
       for (int j = 0; j < D / 32; ++j) qf[j] = *(const f16x8*)(Q + (row + i16) * D + 32 * j + 8 * g);
     }
   };
+  if constexpr (!ONE) load_q(0);
   for (int flat = tid; flat < SK * (D / 8); flat += 256) {
     const int r = flat / (D / 8), u = flat % (D / 8);
     const int off = r * ROW_BYTES + (swz(r, u) << 4);
     *(u32x4*)(&k_lds[off]) = *(const u32x4*)(K + r * D + u * 8);
     *(u32x4*)(&v_lds[off]) = *(const u32x4*)(V + r * D + u * 8);
   }
-  // After K and V: loads return in order, so Q's first, in pieces of 64 bytes,
-  // would hold up the whole workgroup's tile (H4 S128 5.62 us, so 5.23; H32 S1024
-  // 8.8, so 7.95).
-  load_q(0);
+  if constexpr (ONE) load_q(0);
   __syncthreads();
 
   const int ra = sigma(i16);
@@ -1182,9 +1187,9 @@ extern "C" int launch_simple_attention(void* stream, const void* Q, const void* 
     }
   }
   const int64_t groups = (tiles + steps - 1) / steps;
-  hipLaunchKernelGGL(simple_attention_kernel, dim3((unsigned)(groups * H)), dim3(256), 0, (hipStream_t)stream,
-                     (const _Float16*)Q, (const _Float16*)K, (const _Float16*)V, (_Float16*)O, S, (int32_t)groups,
-                     (int32_t)steps);
+  const auto kernel = steps == 1 ? simple_attention_kernel<true> : simple_attention_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * H)), dim3(256), 0, (hipStream_t)stream, (const _Float16*)Q,
+                     (const _Float16*)K, (const _Float16*)V, (_Float16*)O, S, (int32_t)groups, (int32_t)steps);
   return (int)hipGetLastError();
 }
 
